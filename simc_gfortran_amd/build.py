@@ -3,8 +3,8 @@
     python -m simc_gfortran_amd.build
 
 Steps: generate the COSY polynomial code from data/maps (gen_cosy.py), then
-compile the HIP kernels, the output formats and the host map reader into one
-shared library;
+compile the HIP kernels (one unit per kernel family, in parallel), the output
+formats and the host map reader into one shared library;
 build the per-event Fortran-ABI drop-in libsimc_dropin.so on top of it; and,
 when a Fortran compiler is present, compile the Fortran module simc_gpu and
 the Fortran test programs of tests/fortran against both libraries.
@@ -14,6 +14,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(PKG)
@@ -31,9 +32,44 @@ ARCH = os.environ.get("SIMC_OFFLOAD_ARCH", "gfx950")
 # -ffp-contract=off: only the explicit FMAs of the generated polynomials fuse,
 # so every other expression rounds exactly as the reference's does.
 # -packed-fp32-ops off: no v_pk_*_f32 generation.
-HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
+HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
              "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-result"]
+
+# Compilation units: simc_kernels.hip once per kernel family (see its head),
+# so that the families compile in parallel, and the other sources.
+RNGS = {"tape": "TapeStream", "philox": "PhiloxStream", "lane": "PhiloxLaneStream"}
+ARMS = {"hms": "SIMC_ARM_HMS", "shms": "SIMC_ARM_SHMS", "sos": "SIMC_ARM_SOS", "hrs": "SIMC_ARM_HRSR"}
+PARTS = {f"stage_{a}_{r}": ("simc_kernels.hip", [f"-DSIMC_PART_ARM={av}", f"-DSIMC_PART_RNG={rv}"])
+         for a, av in ARMS.items() for r, rv in RNGS.items()}
+PARTS.update({f"adjoint_{a}": ("simc_kernels.hip", [f"-DSIMC_PART_ADJOINT={ARMS[a]}"]) for a in ("hms", "shms")})
+PARTS.update({"rad_tape": ("simc_kernels.hip", ["-DSIMC_PART_RAD=TapeStream"]),
+              "rad_philox": ("simc_kernels.hip", ["-DSIMC_PART_RAD=PhiloxStreamT<kGenTag>"]),
+              "main": ("simc_kernels.hip", []), "io": ("simc_io.hip", []), "maps": ("simc_maps.cpp", [])})
+JOBS = min(8, int(os.environ.get("MAX_JOBS", os.cpu_count() or 8)))
+
+
+def compile_parts(parts, verbose: bool = True):
+    """The parts' object files, compiled JOBS at a time."""
+    def one(item):
+        name, (src, defs) = item
+        obj = os.path.join(GEN, name + ".o")
+        cmd = [HIPCC, *HIP_FLAGS, *defs, "-I", GEN, "-I", CSRC, "-I", os.path.join(REPO, "include"),
+               "-c", os.path.join(CSRC, src), "-o", obj]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.run(cmd, check=True)
+        return obj
+    with ThreadPoolExecutor(JOBS) as pool:
+        return list(pool.map(one, parts.items()))
+
+
+def link(objs, verbose: bool = True):
+    cmd = [HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", LIB + ".tmp"]
+    if verbose:
+        print(" ".join(cmd))
+    subprocess.run(cmd, check=True)
+    os.replace(LIB + ".tmp", LIB)
 
 
 def build(verbose: bool = True) -> str:
@@ -44,14 +80,8 @@ def build(verbose: bool = True) -> str:
     if verbose:
         print("gen_cosy:", summary)
     gen_hut(verbose)
-    srcs = [os.path.join(CSRC, "simc_kernels.hip"), os.path.join(CSRC, "simc_io.hip"),
-            os.path.join(CSRC, "simc_maps.cpp")]
-    cmd = [HIPCC, *HIP_FLAGS, "-I", GEN, "-I", CSRC, "-I", os.path.join(REPO, "include"),
-           *srcs, "-o", LIB + ".tmp"]
-    if verbose:
-        print(" ".join(cmd))
-    subprocess.run(cmd, check=True)
-    os.replace(LIB + ".tmp", LIB)
+    objs = compile_parts(PARTS, verbose)
+    link(objs, verbose)
     build_dropin(verbose)
     build_fortran(verbose)
     return LIB

@@ -33,7 +33,19 @@
 
 using namespace simcdev;
 
-namespace {
+// This file is compiled once per kernel family (build.py), so that the
+// families build in parallel:
+//   SIMC_PART_ARM, SIMC_PART_RNG  the stage kernels of one arm and one random stream
+//   SIMC_PART_ADJOINT             the adjoint's transport and reconstruction passes of one arm
+//   SIMC_PART_RAD                 the radiative generator of one random stream
+//   none of them                  the remaining kernels and the C ABI
+// Each family is reached through a launcher declared for all parts and
+// defined in its own.
+#if !defined(SIMC_PART_ARM) && !defined(SIMC_PART_ADJOINT) && !defined(SIMC_PART_RAD)
+#define SIMC_PART_MAIN
+#endif
+
+namespace simck {
 
 constexpr int kHistBins = 256;
 constexpr int kBlock = 256;  // threads per workgroup (one event each)
@@ -931,6 +943,44 @@ __global__ __launch_bounds__(kBlock) void recon_list_kernel(KArgs a, Queue acc)
     reconstruct_event<ARM>(a, event_id(a, S, s, li).off);
 }
 
+// The four kernels of one launch of arm ARM on stream st: steps [first, coll)
+// over the inputs, [coll, hut) and [hut, end) over the survivors, then the
+// reconstruction of the accepted list acc.  ev: five events marking the
+// kernels' boundaries, or nullptr.
+template <int ARM, class R>
+hipError_t launch_arm(bool rare, const KArgs& a, const Queue& q1, const Queue& q2, const Queue& acc, int32_t first,
+                      int32_t coll, int32_t hut, hipStream_t st, hipEvent_t* ev);
+
+#ifdef SIMC_PART_ARM
+template <int ARM, class R, bool RARE>
+hipError_t launch_variant(const KArgs& a, const Queue& q1, const Queue& q2, const Queue& acc, int32_t first,
+                          int32_t coll, int32_t hut, hipStream_t st, hipEvent_t* ev)
+{
+    const dim3 G((a.count + kBlock - 1) / kBlock), B(kBlock);
+    hipError_t e = ev ? hipEventRecord(ev[0], st) : hipSuccess;
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((stage_kernel<ARM, R, RARE, STAGE_MAGNETS, false, true>), G, B, 0, st, a, q2, q1, first, coll);
+    if (ev && (e = hipEventRecord(ev[1], st)) != hipSuccess) return e;
+    hipLaunchKernelGGL((stage_kernel<ARM, R, RARE, STAGE_MAGNETS, true, true>), G, B, 0, st, a, q1, q2, coll, hut);
+    if (ev && (e = hipEventRecord(ev[2], st)) != hipSuccess) return e;
+    hipLaunchKernelGGL((stage_kernel<ARM, R, RARE, STAGE_HUT, true, true>), G, B, 0, st, a, q2, acc, hut, 0x7fffffff);
+    if (ev && (e = hipEventRecord(ev[3], st)) != hipSuccess) return e;
+    hipLaunchKernelGGL((recon_list_kernel<ARM>), G, B, 0, st, a, acc);
+    if (ev && (e = hipEventRecord(ev[4], st)) != hipSuccess) return e;
+    return hipGetLastError();
+}
+template <int ARM, class R>
+hipError_t launch_arm(bool rare, const KArgs& a, const Queue& q1, const Queue& q2, const Queue& acc, int32_t first,
+                      int32_t coll, int32_t hut, hipStream_t st, hipEvent_t* ev)
+{
+    return rare ? launch_variant<ARM, R, true>(a, q1, q2, acc, first, coll, hut, st, ev)
+                : launch_variant<ARM, R, false>(a, q1, q2, acc, first, coll, hut, st, ev);
+}
+template hipError_t launch_arm<SIMC_PART_ARM, SIMC_PART_RNG>(bool, const KArgs&, const Queue&, const Queue&,
+                                                             const Queue&, int32_t, int32_t, int32_t, hipStream_t,
+                                                             hipEvent_t*);
+#endif
+
 // ---------------------------------------------------------------------------
 // Adjoint form: loss and gradients of an optics fit over a fixed set of
 // events, with the events' random draws replayed (their Philox streams or
@@ -978,6 +1028,7 @@ struct AdjArgs {
 };
 constexpr int kAdjTermsPerLane = 2;   // n_terms <= 512
 
+#ifdef SIMC_PART_MAIN
 __global__ void select_events(const uint8_t* mask, uint32_t n, uint32_t* sel, uint32_t* n_sel)
 {
     __shared__ uint32_t wave_n[kBlock / 64];
@@ -1000,6 +1051,7 @@ __global__ void select_events(const uint8_t* mask, uint32_t n, uint32_t* sel, ui
         sel[slot] = i;
     }
 }
+#endif
 
 // The step program of one event with tangents, up to the track fit.
 // Returns false when a hit of the fit is exactly zero (LFIT would skip it and
@@ -1258,6 +1310,7 @@ __global__ __launch_bounds__(kBlock) void adjoint_recon_kernel(AdjArgs a)
 // its terms' monomials from the table.  Sums go to the device per workgroup.
 constexpr int kAdjTile = 128;
 constexpr int kAdjMaxExp = 6;
+#ifdef SIMC_PART_MAIN
 __global__ __launch_bounds__(kBlock) void adjoint_coef_kernel(AdjArgs a)
 {
     __shared__ double pw[kAdjTile][5][kAdjMaxExp + 1];
@@ -1340,6 +1393,21 @@ __global__ void zero_u64(unsigned long long* p, uint32_t n)
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0ull;
 }
+#endif
+
+// The adjoint's passes 1 and 2 over `blocks` workgroups.
+template <int ARM>
+void launch_adjoint(bool tape, unsigned blocks, hipStream_t st, const AdjArgs& a);
+#ifdef SIMC_PART_ADJOINT
+template <int ARM>
+void launch_adjoint(bool tape, unsigned blocks, hipStream_t st, const AdjArgs& a)
+{
+    if (tape) hipLaunchKernelGGL((adjoint_kernel<ARM, TapeStream>), dim3(blocks), dim3(kBlock), 0, st, a);
+    else hipLaunchKernelGGL((adjoint_kernel<ARM, PhiloxStream>), dim3(blocks), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((adjoint_recon_kernel<ARM>), dim3(blocks), dim3(kBlock), 0, st, a);
+}
+template void launch_adjoint<SIMC_PART_ADJOINT>(bool, unsigned, hipStream_t, const AdjArgs&);
+#endif
 
 template <int ARM>
 __global__ __launch_bounds__(256) void recon_kernel(int64_t n, const double* coef, const uint32_t* gen,
@@ -1529,6 +1597,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
     if (a.used) a.used[i] = g.overflow ? -1 : g.used();
 }
 
+template <class R>
+void launch_gen_hep_rad(dim3 G, dim3 B, hipStream_t st, const GenRadArgs& a);
+#ifdef SIMC_PART_RAD
+template <class R>
+void launch_gen_hep_rad(dim3 G, dim3 B, hipStream_t st, const GenRadArgs& a)
+{
+    hipLaunchKernelGGL((gen_hep_rad_kernel<R>), G, B, 0, st, a);
+}
+template void launch_gen_hep_rad<SIMC_PART_RAD>(dim3, dim3, hipStream_t, const GenRadArgs&);
+#endif
+
+#ifdef SIMC_PART_MAIN
 // ---------------------------------------------------------------------------
 // Target-field tracking (trg_track.f).  Each workgroup stages the field map
 // (2 x 51 x 51 doubles, 41.6 KB) in LDS; one event per lane.
@@ -1709,10 +1789,18 @@ __global__ __launch_bounds__(256) void field_to_search(FieldToArgs a)
 }
 
 __global__ void zero_u32(uint32_t* p) { p[0] = 0u; }
+#endif
 
+}  // namespace simck
+
+#ifdef SIMC_PART_MAIN
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+using namespace simck;
+
+namespace {
+
 thread_local std::string g_err;
 
 int fail(int code, const std::string& msg)
@@ -2340,42 +2428,20 @@ int launch_stages(simc_ctx* ctx, int arm, bool rare, bool tape, const KArgs& a, 
     const int32_t coll = ctx->coll_pc[ai], hut = ctx->hut_pc[ai];
     // the leading sieve steps are no-ops in the common variants
     const int32_t first = rare ? 0 : ctx->lead_pc[ai];
-    const dim3 G((a.count + kBlock - 1) / kBlock), B(kBlock);
     // the accepted list of the hut stage reuses queue 1 (consumed by then)
     // with the third counter
     Queue acc = q1;
     acc.count = q1.count + 2;
     hipLaunchKernelGGL(zero_queue_counts, dim3(1), dim3(64), 0, st, q1.count);
-    if (ev) HIPCHK(hipEventRecord(ev[0], st));
-#define LAUNCH3(ARMV, RV, RARE)                                                                             \
-    do {                                                                                                    \
-        hipLaunchKernelGGL((stage_kernel<ARMV, RV, RARE, STAGE_MAGNETS, false, true>), G, B, 0, st, a, q2, q1, \
-                           first, coll);                                                                    \
-        if (ev) HIPCHK(hipEventRecord(ev[1], st));                                                          \
-        hipLaunchKernelGGL((stage_kernel<ARMV, RV, RARE, STAGE_MAGNETS, true, true>), G, B, 0, st, a, q1, q2,  \
-                           coll, hut);                                                                      \
-        if (ev) HIPCHK(hipEventRecord(ev[2], st));                                                          \
-        hipLaunchKernelGGL((stage_kernel<ARMV, RV, RARE, STAGE_HUT, true, true>), G, B, 0, st, a, q2, acc,     \
-                           hut, 0x7fffffff);                                                                \
-        if (ev) HIPCHK(hipEventRecord(ev[3], st));                                                          \
-        hipLaunchKernelGGL((recon_list_kernel<ARMV>), G, B, 0, st, a, acc);                                 \
-        if (ev) HIPCHK(hipEventRecord(ev[4], st));                                                          \
-    } while (0)
-#define LAUNCH1(ARMV, RV) do { if (rare) LAUNCH3(ARMV, RV, true); else LAUNCH3(ARMV, RV, false); } while (0)
-#define LAUNCHR(ARMV)                                                                                       \
-    do {                                                                                                    \
-        if (tape) LAUNCH1(ARMV, TapeStream);                                                                \
-        else if (lane_key) LAUNCH1(ARMV, PhiloxLaneStream);                                                 \
-        else LAUNCH1(ARMV, PhiloxStream);                                                                   \
-    } while (0)
+#define LAUNCHR(ARMV)                                                                                          \
+    HIPCHK(tape       ? (launch_arm<ARMV, TapeStream>(rare, a, q1, q2, acc, first, coll, hut, st, ev))         \
+           : lane_key ? (launch_arm<ARMV, PhiloxLaneStream>(rare, a, q1, q2, acc, first, coll, hut, st, ev))   \
+                      : (launch_arm<ARMV, PhiloxStream>(rare, a, q1, q2, acc, first, coll, hut, st, ev)))
     if (arm == SIMC_ARM_HMS) LAUNCHR(SIMC_ARM_HMS);
     else if (arm == SIMC_ARM_SOS) LAUNCHR(SIMC_ARM_SOS);
     else if (is_hrs(arm)) LAUNCHR(SIMC_ARM_HRSR);  // one kernel family for both HRS arms (their tables differ)
     else LAUNCHR(SIMC_ARM_SHMS);
 #undef LAUNCHR
-#undef LAUNCH1
-#undef LAUNCH3
-    HIPCHK(hipGetLastError());
     return SIMC_OK;
 }
 
@@ -3251,8 +3317,8 @@ int simc_gen_hep_rad(simc_ctx* ctx, const simc_target* t, const simc_hep_setting
         a.ok = out->ok ? out->ok + at : nullptr;
         a.used = out->used ? out->used + at : nullptr;
         const dim3 G((unsigned)((m + 255) / 256)), B(256);
-        if (rng->kind == SIMC_RNG_TAPE) hipLaunchKernelGGL((gen_hep_rad_kernel<TapeStream>), G, B, 0, st, a);
-        else hipLaunchKernelGGL((gen_hep_rad_kernel<PhiloxStreamT<kGenTag>>), G, B, 0, st, a);
+        if (rng->kind == SIMC_RNG_TAPE) launch_gen_hep_rad<TapeStream>(G, B, st, a);
+        else launch_gen_hep_rad<PhiloxStreamT<kGenTag>>(G, B, st, a);
         HIPCHK(hipGetLastError());
     }
     return SIMC_OK;
@@ -3807,17 +3873,8 @@ int simc_adjoint_run(simc_ctx* ctx, int arm, const simc_settings* s, const simc_
     hipLaunchKernelGGL(zero_queue_counts, dim3(1), dim3(64), 0, st, ctx->d_nsel);
     const unsigned blocks = (unsigned)((n + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(select_events, dim3(blocks), dim3(kBlock), 0, st, mask, (uint32_t)n, ctx->d_sel, ctx->d_nsel);
-#define ADJ(ARMV, RV) hipLaunchKernelGGL((adjoint_kernel<ARMV, RV>), dim3(blocks), dim3(kBlock), 0, st, a)
-    if (arm == SIMC_ARM_HMS) {
-        if (tape) ADJ(SIMC_ARM_HMS, TapeStream); else ADJ(SIMC_ARM_HMS, PhiloxStream);
-    } else {
-        if (tape) ADJ(SIMC_ARM_SHMS, TapeStream); else ADJ(SIMC_ARM_SHMS, PhiloxStream);
-    }
-#undef ADJ
-    if (arm == SIMC_ARM_HMS)
-        hipLaunchKernelGGL((adjoint_recon_kernel<SIMC_ARM_HMS>), dim3(blocks), dim3(kBlock), 0, st, a);
-    else
-        hipLaunchKernelGGL((adjoint_recon_kernel<SIMC_ARM_SHMS>), dim3(blocks), dim3(kBlock), 0, st, a);
+    if (arm == SIMC_ARM_HMS) launch_adjoint<SIMC_ARM_HMS>(tape, blocks, st, a);
+    else launch_adjoint<SIMC_ARM_SHMS>(tape, blocks, st, a);
     const unsigned cgrid = std::min<unsigned>((unsigned)((n + kAdjTile - 1) / kAdjTile), (unsigned)ctx->n_cu * 4u);
     hipLaunchKernelGGL(adjoint_coef_kernel, dim3(cgrid), dim3(kBlock), 0, st, a);
     hipLaunchKernelGGL(adjoint_finish, dim3((nc + 255) / 256), dim3(256), 0, st, grad_coef, nc, out9, ctx->d_nsel);
@@ -4055,3 +4112,4 @@ int64_t simc_poly_flops_full(simc_ctx* ctx, int arm)
 }
 
 }  // extern "C"
+#endif  // SIMC_PART_MAIN
