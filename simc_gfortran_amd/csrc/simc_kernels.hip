@@ -756,9 +756,33 @@ __device__ __forceinline__ void finish_event(const KArgs& a, uint32_t off, int s
 }
 
 // Stop-code counts: the workgroup's LDS histogram serves the setting of its
-// first event; events of other settings (at setting boundaries) count
-// directly in device memory.
-__device__ __forceinline__ void count_stop(const KArgs& a, unsigned* hist, uint32_t s_block, uint32_t s, int bin,
+// first event; events of other settings count directly in device memory.
+// Past the first stage a workgroup holds survivors of several neighbouring
+// settings (queue slots go to workgroups in the order they finish), and most
+// of them share one bin (accepted), so the lanes of one counter are added in
+// the wavefront first: one atomic per counter and wavefront instead of one
+// per event, which serialised on a few addresses (64 settings of two
+// arms, 2e7 events: 13.6 -> 9.2 ms for the whole batch).
+__device__ __forceinline__ void count_stop(const KArgs& a, unsigned* hist, uint32_t s_block, uint32_t s, int bin)
+{
+    if (s == s_block) {
+        atomicAdd(&hist[bin], 1u);
+        return;
+    }
+    const uint32_t key = s * (uint32_t)kHistSlots + (uint32_t)bin;
+    for (bool counted = false; !counted;) {
+        const uint32_t k0 = __builtin_amdgcn_readfirstlane(key);
+        if (key == k0) {
+            counted = true;
+            const uint64_t lanes = __ballot(1);
+            if (__builtin_amdgcn_mbcnt_hi((uint32_t)(lanes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)lanes, 0)) == 0)
+                atomicAdd(&a.hist[(size_t)setting_of(a, s).hist * kHistSlots + bin], (unsigned long long)__popcll(lanes));
+        }
+    }
+}
+
+// Collimator slit hits: the event's own count of a bin.
+__device__ __forceinline__ void count_slit(const KArgs& a, unsigned* hist, uint32_t s_block, uint32_t s, int bin,
                                            unsigned n)
 {
     if (s == s_block) atomicAdd(&hist[bin], n);
@@ -867,17 +891,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2
         if (STAGE == STAGE_HUT) {
             // TO_Q: accepted events go to the reconstruction list
             finish_event<ARM, TO_Q>(a, e.off, st, used, t, resmult);
-            count_stop(a, hist, s_block, s, st, 1u);
+            count_stop(a, hist, s_block, s, st);
             survivor = TO_Q && st == ST_OK;
         } else if (TO_Q && st == ST_OK) {
             survivor = true;
         } else {
             finish_event<ARM>(a, e.off, st, used, t, resmult);
-            count_stop(a, hist, s_block, s, st, 1u);
+            count_stop(a, hist, s_block, s, st);
         }
         if (coll_cnt[0] | coll_cnt[1] | coll_cnt[2]) {
             for (int k = 0; k < 3; ++k)
-                if (coll_cnt[k]) count_stop(a, hist, s_block, s, kHistBins + k, coll_cnt[k]);
+                if (coll_cnt[k]) count_slit(a, hist, s_block, s, kHistBins + k, coll_cnt[k]);
         }
     }
 
