@@ -769,15 +769,15 @@ __device__ __forceinline__ void count_stop(const KArgs& a, unsigned* hist, uint3
         atomicAdd(&hist[bin], 1u);
         return;
     }
+    // each turn serves the lanes that share the first remaining lane's key
+    // (the ballot before the branch: inside it the compiler may move the code
+    // past the loop, where other lanes have joined)
     const uint32_t key = s * (uint32_t)kHistSlots + (uint32_t)bin;
     for (bool counted = false; !counted;) {
-        const uint32_t k0 = __builtin_amdgcn_readfirstlane(key);
-        if (key == k0) {
-            counted = true;
-            const uint64_t lanes = __ballot(1);
-            if (__builtin_amdgcn_mbcnt_hi((uint32_t)(lanes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)lanes, 0)) == 0)
-                atomicAdd(&a.hist[(size_t)setting_of(a, s).hist * kHistSlots + bin], (unsigned long long)__popcll(lanes));
-        }
+        counted = key == (uint32_t)__builtin_amdgcn_readfirstlane(key);
+        const uint64_t same = __ballot(counted);
+        if (counted && __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0)) == 0)
+            atomicAdd(&a.hist[(size_t)setting_of(a, s).hist * kHistSlots + bin], (unsigned long long)__popcll(same));
     }
 }
 
