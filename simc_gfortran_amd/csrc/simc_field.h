@@ -14,53 +14,85 @@ namespace simcdev {
 constexpr int kTrgN = 51;                 // nz = nr = 51, trg_track.f:257-258
 constexpr int kTrgNodes = kTrgN * kTrgN;  // B(iz, ir) at [ir * 51 + iz]
 
-// The map of one launch: B_z, B_r (LDS) and the field angle of the arm
+// One LDS entry of the staged map: B_z and B_r of a node and their
+// differences to the next node in z (the subtraction of the bilinear
+// interpolation, formed once per node instead of at every evaluation).
+// 32 bytes: a node is two 16-byte reads.  The last column serves as a next
+// node only, so 50 x 51 entries are kept: 81,600 bytes, twice in a CU's LDS.
+constexpr int kTrgNz = kTrgN - 1;
+constexpr int kTrgStaged = kTrgNz * kTrgN;  // entry (iz, ir) at [ir * kTrgNz + iz]
+struct __attribute__((aligned(16))) TrgNode {
+    double bz, dbz, br, dbr;
+};
+
+// The map of one launch (LDS) and the field angle of the arm
 // (sin, cos of theta * pi/180 with pi = 3.141592653, trg_track.f:271-281).
 struct TrgMap {
-    const double* bz;
-    const double* br;
+    const TrgNode* node;
     double stht, ctht;
 };
 
+// Square root by one coupled (Goldschmidt) iteration from the hardware's
+// reciprocal square root (2^-24) and one residual correction (Markstein);
+// `y` receives 1 / sqrt(s) to 2^-47, enough for div_by's residual to round a
+// quotient.  Before their last rounding both results are within 2^-42 ulp;
+// for s in [2^-900, 2^1000] they equalled sqrt(s) and a / sqrt(s) on all of
+// 5e9 samples, without the scaling and special cases of the general forms.
+__device__ __forceinline__ double sqrt_inv(double s, double& y)
+{
+    const double y0 = __builtin_amdgcn_rsq(s);
+    double g = s * y0, h = 0.5 * y0;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    y = h + h;
+    return __builtin_fma(__builtin_fma(-g, g, s), h, g);
+}
+// a / r from y = 1 / r to 2^-47
+__device__ __forceinline__ double div_by(double a, double r, double y)
+{
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-r, q, a), y, q);
+}
+
 // trgField, trg_track.f:328-418.  The grid starts at 0 with spacing 2, so
-// zz(i) = 2 (i - 1) and (z - zz(1)) / (zz(2) - zz(1)) = z / 2 exactly.
-// Points at |z'| or r >= 200 cm are outside the grid (field 0) before the
-// integer conversion, which keeps it in range.
+// zz(i) = 2 (i - 1), (z - zz(1)) / (zz(2) - zz(1)) = z / 2 exactly, and the
+// interpolation's (z - zz(i)) / 2 is the fractional part of z / 2, exact too.
+// A point is inside the grid when floor(z / 2) + 2 <= 51, that is z < 100 cm,
+// and r likewise (r^2 < 10^4: no double just below it has the root 100).
 __device__ __forceinline__ void trg_field(const TrgMap& M, double x0, double x1, double x2, double& B0,
                                           double& B1, double& B2)
 {
     const double y1 = M.stht * x2 + M.ctht * x1;
     const double y2 = M.ctht * x2 - M.stht * x1;
-    const double z = fabs(y2);
-    const double r = sqrt(x0 * x0 + y1 * y1);
+    const double s = x0 * x0 + y1 * y1;
     B0 = 0.0;
     B1 = 0.0;
     B2 = 0.0;
-    if (!(z < 200.0) || !(r < 200.0)) return;
-    const int i = (int)(z / 2.0) + 1;
-    const int j = (int)(r / 2.0) + 1;
-    if ((i + 1 > kTrgN) || (i < 1) || (j + 1 > kTrgN) || (j < 1)) return;
-    const int i0 = i - 1, j0 = j - 1;
-    const double az = ((z - 2.0 * (double)i0) / 2.0);
-    const double ar = ((r - 2.0 * (double)j0) / 2.0);
-    const double* bz = M.bz + j0 * kTrgN + i0;
-    double a0 = az * (bz[1] - bz[0]) + bz[0];
-    double a1 = az * (bz[kTrgN + 1] - bz[kTrgN]) + bz[kTrgN];
-    const double Bz = (ar * (a1 - a0) + a0);
-    if (r > 0.0) {
-        const double* br = M.br + j0 * kTrgN + i0;
-        a0 = az * (br[1] - br[0]) + br[0];
-        a1 = az * (br[kTrgN + 1] - br[kTrgN]) + br[kTrgN];
-        double b = (ar * (a1 - a0) + a0) / r;
-        if (y2 < 0.0) b = -b;
-        const double Bx = b * x0, By = b * y1;
-        B0 = Bx;
-        B1 = -M.stht * Bz + M.ctht * By;
-        B2 = M.ctht * Bz + M.stht * By;
-    } else {
-        B1 = -M.stht * Bz;
-        B2 = M.ctht * Bz;
+    if (!(fabs(y2) < 100.0) || !(s < 10000.0)) return;
+    double rinv;
+    double r = sqrt_inv(s, rinv);
+    const bool axis = s < 0x1p-900;  // on the field axis
+    if (__builtin_expect(axis, 0)) {
+        r = sqrt(s);
+        rinv = r > 0.0 ? 1.0 / r : 0.0;  // the quotient below is 0 for r = 0
     }
+    const double zh = fabs(y2) * 0.5, rh = r * 0.5;
+    const double az = __builtin_amdgcn_fract(zh), ar = __builtin_amdgcn_fract(rh);
+    const TrgNode* p = M.node + ((int)rh * kTrgNz + (int)zh);
+    const TrgNode n0 = p[0], n1 = p[kTrgNz];
+    double a0 = az * n0.dbz + n0.bz;
+    double a1 = az * n1.dbz + n1.bz;
+    const double Bz = (ar * (a1 - a0) + a0);
+    a0 = az * n0.dbr + n0.br;
+    a1 = az * n1.dbr + n1.br;
+    const double num = (ar * (a1 - a0) + a0);
+    double b = div_by(num, r, rinv);
+    if (y2 < 0.0) b = -b;
+    const double Bx = b * x0, By = b * y1;
+    B0 = Bx;
+    B1 = -M.stht * Bz + M.ctht * By;
+    B2 = M.ctht * Bz + M.stht * By;
 }
 
 // trgDeriv, trg_track.f:423-459: (v, (v x B) * factor); the integral terms
@@ -177,9 +209,12 @@ __device__ __forceinline__ bool track_from_tgt(const TrgMap& M, double& x, doubl
     double vT[6];
     trg_start(vT, x, y, z, dx, dy, vel, true);
     bool ok = true;
-    trg_track_to_plane(M, vT, eng, 1., 0., 0., 1., 0., ok);
-    ok = true;
-    trg_track_to_plane(M, vT, eng, 1., 0., 0., 1., -100., ok);
+    // one copy of the search for both planes (its code is long)
+#pragma unroll 1
+    for (int leg = 0; leg < 2; ++leg) {
+        ok = true;
+        trg_track_to_plane(M, vT, eng, 1., 0., 0., 1., leg ? -100. : 0., ok);
+    }
     x = vT[0];
     y = vT[1];
     z = vT[2];

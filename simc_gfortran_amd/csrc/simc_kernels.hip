@@ -1635,7 +1635,12 @@ template void launch_gen_hep_rad<SIMC_PART_RAD>(dim3, dim3, hipStream_t, const G
 #ifdef SIMC_PART_MAIN
 // ---------------------------------------------------------------------------
 // Target-field tracking (trg_track.f).  Each workgroup stages the field map
-// (2 x 51 x 51 doubles, 41.6 KB) in LDS; one event per lane.
+// with its differences (50 x 51 entries of 32 bytes, 82 KB: two workgroups per
+// CU) in LDS; one event per lane.  Bound by VALU issue: an RK4 step is about 420
+// instructions (550 with the general square root and division, the map's
+// subtractions and the grid tests on integers), 4.3 cycles each at four
+// wavefronts per SIMD (three before).  1e6 vertices to z = 100 cm: 1.68 ->
+// 1.19 ms.
 // ---------------------------------------------------------------------------
 struct FieldFromArgs {
     const double* map;  // B_z nodes, then B_r nodes
@@ -1647,19 +1652,37 @@ struct FieldFromArgs {
     uint8_t* ok;
 };
 
-__device__ __forceinline__ void stage_field_map(double* s, const double* map)
+__device__ __forceinline__ void stage_field_map(TrgNode* s, const double* map)
 {
-    for (int k = threadIdx.x; k < 2 * kTrgNodes; k += blockDim.x) s[k] = map[k];
+    for (int k = threadIdx.x; k < kTrgStaged; k += blockDim.x) {
+        const double* b = map + (k / kTrgNz) * kTrgN + k % kTrgNz;
+        TrgNode v;
+        v.bz = b[0];
+        v.dbz = b[1] - v.bz;
+        v.br = b[kTrgNodes];
+        v.dbr = b[kTrgNodes + 1] - v.br;
+        s[k] = v;
+    }
     __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void field_from_kernel(FieldFromArgs a)
+// Workgroup size of the field kernels for n events (64 .. kFieldBlock): one
+// workgroup per CU while the events fit that way, so that a small run's
+// wavefronts spread over all SIMDs instead of filling a few CUs.
+constexpr int kFieldBlock = 512;
+inline uint32_t field_block(uint64_t n, int n_cu)
 {
-    __shared__ double s[2 * kTrgNodes];
+    const uint64_t per_cu = (n + n_cu - 1) / (uint64_t)n_cu;
+    return (uint32_t)std::min<uint64_t>(kFieldBlock, std::max<uint64_t>(64, (per_cu + 63) / 64 * 64));
+}
+
+__global__ __launch_bounds__(kFieldBlock) __attribute__((amdgpu_waves_per_eu(4))) void field_from_kernel(FieldFromArgs a)
+{
+    __shared__ TrgNode s[kTrgStaged];
     stage_field_map(s, a.map);
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n) return;
-    const TrgMap M{s, s + kTrgNodes, a.stht, a.ctht};
+    const TrgMap M{s, a.stht, a.ctht};
     double x = a.x[i], y = a.y[i], z = a.z[i], dx = a.dx[i], dy = a.dy[i];
     const bool ok = track_from_tgt(M, x, y, z, dx, dy, a.mom[i], a.mass);
     a.x[i] = x;
@@ -1670,7 +1693,7 @@ __global__ __launch_bounds__(256) void field_from_kernel(FieldFromArgs a)
     if (a.ok) a.ok[i] = ok ? 1 : 0;
 }
 
-// track_to_tgt (trg_track.f:738-876) in rounds.  The reference's loop
+// track_to_tgt (trg_track.f:738-876): rounds, then a finish.  The reference's loop
 // alternates plane searches (RK4, a few hundred steps) with the arm's
 // reconstruction, and events leave it after 1 to 10 iterations.  One lane
 // per event through the whole loop would run every wave as long as its
@@ -1679,8 +1702,9 @@ __global__ __launch_bounds__(256) void field_from_kernel(FieldFromArgs a)
 // iteration's searches up to the reconstruction; then, per round, a
 // reconstruction kernel and a search kernel run over the list of events
 // still iterating, the search kernel appending the events that continue to
-// the next round's list.  Per event the operations and their order are the
-// reference's, so the rounds change nothing in the results.
+// the next round's list; the events left after a few rounds go to
+// field_to_finish.  Per event the operations and their order are the
+// reference's, so neither changes anything in the results.
 struct FieldToArgs {
     const double* map;
     double stht, ctht;
@@ -1749,13 +1773,13 @@ __device__ __forceinline__ void field_to_iterate(const TrgMap& M, const FieldToA
 }
 
 // Round 0: the first search from z = 100 cm to the beam plane (:768-787).
-__global__ __launch_bounds__(256) void field_to_start(FieldToArgs a)
+__global__ __launch_bounds__(kFieldBlock) __attribute__((amdgpu_waves_per_eu(4))) void field_to_start(FieldToArgs a)
 {
-    __shared__ double s[2 * kTrgNodes];
+    __shared__ TrgNode s[kTrgStaged];
     stage_field_map(s, a.map);
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n) return;
-    const TrgMap M{s, s + kTrgNodes, a.stht, a.ctht};
+    const TrgMap M{s, a.stht, a.ctht};
     const double delta = a.delta[i], y = a.y[i], dx = a.dx[i], dy = a.dy[i];
     const double fry = a.fry[i];
     const double mom = a.mom[i];
@@ -1791,16 +1815,16 @@ __global__ __launch_bounds__(256) void field_to_recon(FieldToArgs a)
 
 // A round's search back to the beam plane from the reconstructed track
 // (:848-865), then the loop test and the next searches.
-__global__ __launch_bounds__(256) void field_to_search(FieldToArgs a)
+__global__ __launch_bounds__(kFieldBlock) __attribute__((amdgpu_waves_per_eu(4))) void field_to_search(FieldToArgs a)
 {
-    __shared__ double s[2 * kTrgNodes];
+    __shared__ TrgNode s[kTrgStaged];
     const uint32_t count = *a.count_in;
-    if (blockIdx.x * 256u >= count) return;  // the whole workgroup is past the list
+    if (blockIdx.x * blockDim.x >= count) return;  // the whole workgroup is past the list
     stage_field_map(s, a.map);
-    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= count) return;
     const uint32_t i = a.list_in[j];
-    const TrgMap M{s, s + kTrgNodes, a.stht, a.ctht};
+    const TrgMap M{s, a.stht, a.ctht};
     const double delta = a.delta[i], y = a.y[i], dx = a.dx[i], dy = a.dy[i], xx = a.xx[i];
     bool ok = a.st_ok[i] != 0;
     const double mom = a.mom0[i] * (1.e0 + delta / 100.e0);
@@ -1810,6 +1834,83 @@ __global__ __launch_bounds__(256) void field_to_search(FieldToArgs a)
     trg_start(vT, xx + 100. * dx, y + 100. * dy, 100., dx, dy, vel, false);
     trg_track_to_plane(M, vT, eng, 1., 0., -a.ctheta, a.stheta, a.frx[i], ok);
     field_to_iterate(M, a, i, vT, eng, xx, a.delx[i], (int)a.iter[i] + 1, ok);
+}
+
+// What is left of the loop for the events still iterating after the rounds:
+// the whole loop per event, in one launch.  A late event's searches take up
+// to 800 steps where the mean is 100, and in rounds every round waits for its
+// own longest search; here the searches of one event follow one another
+// without waiting for the others.  Bound by the longest event's chain of
+// dependent RK4 steps (3,300 of 1.4 us each for 1e5 HMS events, where the
+// mean is 580).  Two lanes per event: both run the reconstruction and the
+// long search (the same values), one each of the two searches to z = 0.
+// Events are dealt out over all wavefronts (event e to wavefront e mod the
+// number of wavefronts), so that few of them share a wavefront's loop.
+constexpr uint32_t kFinishEvents = 256 / 2;  // events a workgroup takes at once
+
+// Rounds before field_to_finish for n events when it takes `cap` at once:
+// none where all fit, else as many as leave about one filling (of 1e5 HMS
+// events 97 % iterate after two rounds, 61, 29, 16 and 10 % after three to
+// six).  Measured in ms with 0, 3, 4, 5, 9 rounds (cap 65,536): 1e3 events
+// 3.6, 3.0, 3.1, 3.4, 4.9; 6e4: 5.5, 6.4, 6.8, 7.9, 9.3; 1e5: 7.9, 6.9, 8.1,
+// 9.9, 13.8; 2e5: 12.6, 9.7, 8.5, 10.0, 16.2; 7e5: -, 24.8, 19.7, 16.9, 18.8.
+// Ten rounds with the same search took 14.3 ms for the 1e5.
+inline int field_rounds(uint64_t n, uint64_t cap) { return n <= cap ? 0 : n <= 2 * cap ? 3 : n <= 4 * cap ? 4 : 5; }
+
+template <int ARM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void field_to_finish(FieldToArgs a)
+{
+    __shared__ TrgNode s[kTrgStaged];
+    const uint32_t count = *a.count_in;
+    const uint32_t n_waves = gridDim.x * (256u / 64u);
+    // wavefronts of a workgroup are numbered gridDim.x apart: the first events go to different CUs
+    const uint32_t wave = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+    if (blockIdx.x >= count) return;  // no event for any wavefront of this workgroup
+    stage_field_map(s, a.map);
+    const TrgMap M{s, a.stht, a.ctht};
+    const bool second = (threadIdx.x & 1u) != 0;
+    for (uint32_t e = wave + ((threadIdx.x & 63u) >> 1) * n_waves; e < count; e += 32u * n_waves) {
+        const uint32_t i = a.list_in[e];
+        EvOut o, r;
+        o.x_fp = a.x_fp[i];
+        o.dx_fp = a.dx_fp[i];
+        o.y_fp = a.y_fp[i];
+        o.dy_fp = a.dy_fp[i];
+        const double fry = a.fry[i], frx = a.frx[i], mom0 = a.mom0[i];
+        double xx = a.xx[i], delx = a.delx[i], vT[6];
+        int n = a.iter[i];
+        bool ok = a.st_ok[i] != 0;
+        for (;;) {
+            recon<ARM>((cdptr)a.coef, (cuptr)a.gen, o, xx, r);
+            double vel, eng;
+            field_energy(mom0 * (1.e0 + r.dpp / 100.e0), a.mass, vel, eng);
+            trg_start(vT, xx + 100. * r.dxdz, r.y + 100. * r.dydz, 100., r.dxdz, r.dydz, vel, false);
+            trg_track_to_plane(M, vT, eng, 1., 0., -a.ctheta, a.stheta, frx, ok);
+            ++n;
+            if (!((delx > .0001) && (n < 10) && ok)) break;
+            // the next iteration's searches (trg_track.f:803-821): of vT by
+            // the first lane, of vT at x = -fry by the second
+            delx = fabs(-fry - vT[0]);
+            if (second) vT[0] = -fry;
+            trg_track_to_plane(M, vT, eng, 1., 0., 0., 1., 0., ok);
+            const double x_other = __shfl_xor(vT[0], 1);
+            const bool ok_other = __shfl_xor((int)ok, 1) != 0;
+            const double x0 = second ? x_other : vT[0];
+            const bool ok0 = second ? ok_other : ok;
+            // the second search runs after a first that succeeded only
+            const double x1 = !ok0 ? -fry : second ? vT[0] : x_other;
+            ok = ok && ok_other;
+            xx = xx + fmin(1., fmax(-1., (x1 - x0)));
+        }
+        if (delx > .2) ok = false;
+        if (!second) {
+            a.delta[i] = r.dpp;
+            a.dy[i] = vT[4] / vT[5];
+            a.dx[i] = vT[3] / vT[5];
+            a.y[i] = vT[1];
+            if (a.ok) a.ok[i] = ok ? 1 : 0;
+        }
+    }
 }
 
 __global__ void zero_u32(uint32_t* p) { p[0] = 0u; }
@@ -3421,6 +3522,7 @@ struct simc_field {
     double* d_map = nullptr;   // B_z nodes, then B_r nodes (2 x 2601)
     double stht[2] = {}, ctht[2] = {};   // [0]: spect -1 (electron arm), [1]: spect +1
     int device = 0;
+    int n_cu = 256;
     std::mutex mu;             // guards the host-pointer staging
     void* d_stage = nullptr;
     size_t stage_bytes = 0;
@@ -3514,6 +3616,7 @@ int simc_field_create(const char* map, double theta_e, double phi_e, double thet
     f->stht[1] = std::sin(theta_p * pi180);
     f->ctht[1] = std::cos(theta_p * pi180);
     if (hipGetDevice(&f->device) != hipSuccess ||
+        hipDeviceGetAttribute(&f->n_cu, hipDeviceAttributeMultiprocessorCount, f->device) != hipSuccess ||
         hipMalloc(&f->d_map, nodes.size() * sizeof(double)) != hipSuccess ||
         hipMemcpy(f->d_map, nodes.data(), nodes.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
         if (f->d_map) (void)hipFree(f->d_map);
@@ -3549,7 +3652,8 @@ int simc_track_from_tgt(const simc_field* f, int spect, int64_t n, double* x, do
     a.mom = mom;
     a.mass = mass;
     a.ok = ok;
-    hipLaunchKernelGGL(field_from_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a);
+    const uint32_t nb = field_block((uint64_t)n, f->n_cu);
+    hipLaunchKernelGGL(field_from_kernel, dim3((uint32_t)((n + nb - 1) / nb)), dim3(nb), 0, (hipStream_t)stream, a);
     HIPCHK(hipGetLastError());
     return SIMC_OK;
 }
@@ -3611,26 +3715,37 @@ int simc_track_to_tgt(simc_ctx* ctx, const simc_field* f, int arm, int spect, in
     a.mass = mass; a.ctheta = ctheta; a.stheta = stheta;
     a.ok = ok;
     const dim3 G((uint32_t)((n + 255) / 256)), B(256);
+    const uint32_t nb = field_block((uint64_t)n, f->n_cu);
+    const dim3 GS((uint32_t)((n + nb - 1) / nb)), BS(nb);
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, st, count);
     a.list_out = list[0];
     a.count_out = count;
-    hipLaunchKernelGGL(field_to_start, G, B, 0, st, a);
-    // at most 10 iterations (trg_track.f:800): after round r every event
-    // still listed has made r + 1 of them
-    for (int r = 0; r < 10; ++r) {
+    hipLaunchKernelGGL(field_to_start, GS, BS, 0, st, a);
+    const uint32_t finish_grid = (uint32_t)f->n_cu * 2u;
+    const int rounds = field_rounds((uint64_t)n, (uint64_t)finish_grid * kFinishEvents);
+#define FOR_ARM(KERNEL, GRID)                                                                              \
+    do {                                                                                                   \
+        if (arm == SIMC_ARM_HMS) hipLaunchKernelGGL(KERNEL<SIMC_ARM_HMS>, GRID, B, 0, st, a);              \
+        else if (arm == SIMC_ARM_SOS) hipLaunchKernelGGL(KERNEL<SIMC_ARM_SOS>, GRID, B, 0, st, a);         \
+        else if (is_hrs(arm)) hipLaunchKernelGGL(KERNEL<SIMC_ARM_HRSR>, GRID, B, 0, st, a);                \
+        else hipLaunchKernelGGL(KERNEL<SIMC_ARM_SHMS>, GRID, B, 0, st, a);                                 \
+    } while (0)
+    for (int r = 0; r <= rounds; ++r) {
         const int in = r & 1;
         a.list_in = list[in];
         a.count_in = count + in;
         a.list_out = list[in ^ 1];
         a.count_out = count + (in ^ 1);
+        if (r == rounds) {
+            FOR_ARM(field_to_finish, dim3(finish_grid));
+            break;
+        }
         hipLaunchKernelGGL(zero_u32, dim3(1), dim3(1), 0, st, a.count_out);
-        if (arm == SIMC_ARM_HMS) hipLaunchKernelGGL(field_to_recon<SIMC_ARM_HMS>, G, B, 0, st, a);
-        else if (arm == SIMC_ARM_SOS) hipLaunchKernelGGL(field_to_recon<SIMC_ARM_SOS>, G, B, 0, st, a);
-        else if (is_hrs(arm)) hipLaunchKernelGGL(field_to_recon<SIMC_ARM_HRSR>, G, B, 0, st, a);
-        else hipLaunchKernelGGL(field_to_recon<SIMC_ARM_SHMS>, G, B, 0, st, a);
-        hipLaunchKernelGGL(field_to_search, G, B, 0, st, a);
+        FOR_ARM(field_to_recon, G);
+        hipLaunchKernelGGL(field_to_search, GS, BS, 0, st, a);
     }
+#undef FOR_ARM
     HIPCHK(hipGetLastError());
     return SIMC_OK;
 }

@@ -169,3 +169,27 @@ def test_empty_inputs(ctx):
     rec = {k: z.clone() for k in ("delta", "y", "dx", "dy")}
     assert F.track_to_tgt(ctx, 1, trk, rec, z, z, z, 938.0, 1.0, 0.0, 1).numel() == 0
     F.close()
+
+
+@pytest.mark.parametrize("n", [1, 65, 65_535, 65_537, 131_073, 262_145])
+def test_to_tgt_same_for_any_number_of_events(ctx, n):
+    """The rounds before the finishing kernel depend on the number of events
+    (none up to 65,536, then 3, 4 and 5 on 256 CUs); an event's result does
+    not: tiles of the golden tracks equal the same tracks run alone."""
+    from simc_gfortran_amd import api
+    g = np.load(os.path.join(HERE, "golden", "field", "to_hms_proton.npz"))
+    F = field_of(api, str(g["map"]), float(g["theta_e"]), float(g["theta_p"]))
+    m = len(g["mom"])
+
+    def run(k):
+        at = np.arange(k) % m
+        trk = {q: dev(g["trk_" + q][at]) for q in ("x_fp", "dx_fp", "y_fp", "dy_fp")}
+        rec = {q: dev(g["in_" + q][at]) for q in ("delta", "y", "dx", "dy")}
+        ok = F.track_to_tgt(ctx, int(g["arm"]), trk, rec, dev(g["frx"][at]), dev(g["fry"][at]), dev(g["mom"][at]),
+                            float(g["mass"]), float(g["ctheta"]), float(g["stheta"]), int(g["spect"]))
+        torch.cuda.synchronize()
+        return dict({q: v.cpu().numpy() for q, v in rec.items()}, ok=ok.cpu().numpy())
+    one, all_ = run(m), run(n)
+    for k in one:
+        np.testing.assert_array_equal(all_[k], one[k][np.arange(n) % m], err_msg=k)
+    F.close()
