@@ -100,6 +100,29 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
     out[0] = c0; out[1] = c1; out[2] = c2; out[3] = c3;
 }
 
+// Square root by one coupled (Goldschmidt) iteration from the hardware's
+// reciprocal square root (2^-24) and one residual correction (Markstein);
+// `y` receives 1 / sqrt(s) to 2^-47, enough for div_by's residual to round a
+// quotient.  Before their last rounding both results are within 2^-42 ulp;
+// for s in [2^-900, 2^1000] they equalled sqrt(s) and a / sqrt(s) on all of
+// 5e9 samples, without the scaling and special cases of the general forms.
+__device__ __forceinline__ double sqrt_inv(double s, double& y)
+{
+    const double y0 = __builtin_amdgcn_rsq(s);
+    double g = s * y0, h = 0.5 * y0;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    y = h + h;
+    return __builtin_fma(__builtin_fma(-g, g, s), h, g);
+}
+// a / r from y = 1 / r to 2^-47
+__device__ __forceinline__ double div_by(double a, double r, double y)
+{
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-r, q, a), y, q);
+}
+
 // ---------------------------------------------------------------------------
 // Elementary functions of the Box-Muller normal generator.  Both are fixed
 // sequences of IEEE operations (explicit fma, exact reductions) over the
@@ -113,22 +136,25 @@ struct __attribute__((aligned(16))) BmLogEntry {
 static __constant__ BmLogEntry kBmLogTab[SIMC_BM_LOG_N] = SIMC_BM_LOG_TABLE;
 static __constant__ double kBmSinCosTab[SIMC_BM_SINCOS_N][2] = SIMC_BM_SINCOS_TABLE;
 
-// Natural logarithm of u in (0, 1) (normal numbers): u = m 2^e with m in
-// [sqrt(1/2), sqrt(2)); c = 1 + k/64 the nearest table point, invc = 1/c to
-// 7 bits, so t = m invc - 1 is exact (|t| < 0.0155); log m = -log(invc) +
-// log1p(t), log1p by its series to t^9 (truncation below 2^-56 relative);
-// then e ln2 in two parts (ln2_hi has 21 significant bits, so e ln2_hi is
-// exact) and the table's two-part -log(invc).
-__device__ __forceinline__ double bm_log(double u)
+// Natural logarithm of u = (w + 1/2) 2^-32: u = m 2^e with m in [sqrt(1/2),
+// sqrt(2)), split on the bits (a 64-bit subtraction of sqrt(1/2)'s, whose
+// exponent field is then e); c = 1 + k/64 the nearest table point, k =
+// rint((m - 1) 64) taken from the low word of one fma onto 1.5 2^52 (an even
+// offset, so ties go the same way); invc = 1/c to 7 bits, so t = m invc - 1
+// is exact (|t| < 0.0155); log m = -log(invc) + log1p(t), log1p by its series
+// to t^9 (truncation below 2^-56 relative); then e ln2 in two parts (ln2_hi
+// has 21 significant bits, so e ln2_hi is exact) and the table's two-part
+// -log(invc).
+__device__ __forceinline__ double bm_log(uint32_t w)
 {
-    double m = __builtin_amdgcn_frexp_mant(u);  // [1/2, 1)
-    int e = __builtin_amdgcn_frexp_exp(u);
-    if (m < 0x1.6a09e667f3bcdp-1) {
-        m = m * 2.0;
-        e = e - 1;
-    }
-    const double kd = rint((m - 1.0) * 64.0);
-    const BmLogEntry L = kBmLogTab[(int)kd + SIMC_BM_LOG_K0];
+    const double u = __builtin_fma((double)w, 0x1p-32, 0x1p-33);  // exact
+    const uint64_t ub = __builtin_bit_cast(uint64_t, u);
+    const int e = (int)(uint32_t)((ub - 0x3fe6a09e667f3bcdull) >> 32) >> 20;
+    const uint32_t mhi = (uint32_t)(ub >> 32) - ((uint32_t)e << 20);
+    const double m = __builtin_bit_cast(double, ((uint64_t)mhi << 32) | (uint32_t)ub);
+    static_assert(SIMC_BM_LOG_K0 == 19, "the table's first point");
+    const double kd = __builtin_fma(m, 64.0, 0x1.8p52 - 64.0 + 20.0);  // low word: k + 20
+    const BmLogEntry L = kBmLogTab[(int)(uint32_t)__builtin_bit_cast(uint64_t, kd) - 1];
     const double t = __builtin_fma(m, (double)L.invc, -1.0);
     double q = 0x1.c71c71c71c71cp-4;                 // 1/9
     q = __builtin_fma(t, q, -0x1p-3);                // -1/8
@@ -143,16 +169,16 @@ __device__ __forceinline__ double bm_log(double u)
     return __builtin_fma(de, 0x1.62e42p-1, L.nhi + (p + __builtin_fma(de, 0x1.fdf473de6af28p-22, (double)L.nlo)));
 }
 
-// sin and cos of 2 pi u for u in [0, 1): x = 64u (exact), k = rint(x),
-// r = x - k in [-1/2, 1/2] (exact), d = r pi/32; sin d and cos d by their
+// sin and cos of 2 pi u for u = (w + 1/2) 2^-32: 64 u = k + r with k =
+// rint(64 u) and r in [-1/2, 1/2], both read off w (its low 26 bits with
+// sign are 2^26 r - 1/2), d = r pi/32 in one fma; sin d and cos d by their
 // Taylor series to d^9 and d^8 (|d| <= pi/64, truncation below 2^-62), then
 // the rotation by the table's sin and cos of 2 pi k/64.
-__device__ __forceinline__ void bm_sincos2pi(double u, double& sn, double& cs)
+__device__ __forceinline__ void bm_sincos2pi(uint32_t w, double& sn, double& cs)
 {
-    const double x = u * 64.0;
-    const double kd = rint(x);
-    const double r = x - kd;
-    const double d = r * 0x1.921fb54442d18p-4;
+    const uint32_t k = (w + (1u << 25)) >> 26;
+    const int rw = (int)(w << 6) >> 6;
+    const double d = __builtin_fma((double)rw, 0x1.921fb54442d18p-30, 0x1.921fb54442d18p-31);
     const double z = d * d;
     double ps = 0x1.71de3a556c734p-19;                 // 1/9!
     ps = __builtin_fma(z, ps, -0x1.a01a01a01a01ap-13);  // -1/7!
@@ -164,10 +190,20 @@ __device__ __forceinline__ void bm_sincos2pi(double u, double& sn, double& cs)
     pc = __builtin_fma(z, pc, 0x1.5555555555555p-5);    // 1/4!
     pc = __builtin_fma(z, pc, -0x1p-1);                 // -1/2
     const double cd = __builtin_fma(z, pc, 1.0);
-    const int k = (int)kd & 63;
     const double sa = kBmSinCosTab[k][0], ca = kBmSinCosTab[k][1];
     sn = __builtin_fma(sa, cd, ca * sd);
     cs = __builtin_fma(ca, cd, -(sa * sd));
+}
+
+// The Box-Muller pair of two words: sqrt(-2 ln u1) (cos 2 pi u2, sin 2 pi u2).
+// -2 ln u1 lies in [2^-32, 46], inside sqrt_inv's range.
+__device__ __forceinline__ void bm_pair(uint32_t w1, uint32_t w2, double& c, double& sn_)
+{
+    double y, sn, cs;
+    const double r = sqrt_inv(-2.0 * bm_log(w1), y);
+    bm_sincos2pi(w2, sn, cs);
+    c = r * cs;
+    sn_ = r * sn;
 }
 
 // TAG is the fourth counter word: streams of different tags are independent
@@ -216,13 +252,17 @@ struct PhiloxStreamT {
             if ((pos & 3u) >= 3u) shift();
         }
     }
-    __device__ __forceinline__ double next()
+    __device__ __forceinline__ uint32_t next_word()
     {
         if ((pos & 3u) == 0) philox4x32_10<LANE_KEY>(pos >> 2, e0, e1, TAG, k0, k1, w);
         ++pos;
         const uint32_t v = w[0];
         shift();
-        return __builtin_fma((double)v, 0x1p-32, 0x1p-33);  // (v + 1/2) 2^-32, exact
+        return v;
+    }
+    __device__ __forceinline__ double next()
+    {
+        return __builtin_fma((double)next_word(), 0x1p-32, 0x1p-33);  // (v + 1/2) 2^-32, exact
     }
     // Normal deviates for the counter-based stream: Box-Muller pairs
     // (u1, u2) -> sqrt(-2 ln u1) (cos 2 pi u2, sin 2 pi u2), both used, the
@@ -238,14 +278,11 @@ struct PhiloxStreamT {
                 if (fabs(pending) <= nsigmax) return pending;
                 continue;
             }
-            const double u1 = next();
-            const double u2 = next();
-            const double r = sqrt(-2.0 * bm_log(u1));
-            double sn, cs;
-            bm_sincos2pi(u2, sn, cs);
-            pending = r * sn;
+            const uint32_t w1 = next_word();
+            const uint32_t w2 = next_word();
+            double g1;
+            bm_pair(w1, w2, g1, pending);
             have = 1;
-            const double g1 = r * cs;
             if (fabs(g1) <= nsigmax) return g1;
         }
     }
@@ -259,13 +296,9 @@ struct PhiloxStreamT {
             b = gauss(99.0);
             return;
         }
-        const double u1 = next();
-        const double u2 = next();
-        const double r = sqrt(-2.0 * bm_log(u1));
-        double sn, cs;
-        bm_sincos2pi(u2, sn, cs);
-        a = r * cs;
-        b = r * sn;
+        const uint32_t w1 = next_word();
+        const uint32_t w2 = next_word();
+        bm_pair(w1, w2, a, b);
         pending = b;
     }
     __device__ __forceinline__ int32_t used() const { return (int32_t)pos; }
@@ -275,39 +308,130 @@ using PhiloxLaneStream = PhiloxStreamT<kPhiloxTag, true>;
 
 // The detector hut's own counter-based stream: uniform k of an event's hut
 // is word k%4 of the Philox block (k/4, event lo, event hi, kHutTag) under
-// the event's key.  Every hut step draws one uniform (resmult) or Box-Muller
-// pairs (both values used, cosine first), so nothing is pending between
-// steps.  The draws depend on launch-uniform flags only: the position is the
-// same in every lane of a wavefront, so block refills and word selection are
+// the event's key.  A hut draws at most one uniform (resmult), before any
+// other, and then Box-Muller pairs (both values used, cosine first), so
+// nothing is pending between steps.  The draws depend on launch-uniform flags
+// only: the position is the same in every lane of a wavefront, so refills are
 // scalar branches.
+//
+// Pairs are formed two at a time, one Philox block, in a function of its own
+// (hut_pairs): inlined at each of the hut's ~100 draws the SHMS hut was 327 KB
+// of straight-line code, five times the instruction cache, and every
+// wavefront streamed it from L2.  The block's first two rounds depend on the
+// lane through the event id alone, so their products are formed once per
+// event (a, h, l below) and the counter's part is scalar.
+struct HutPairs {
+    double a0, b0, a1, b1;
+    uint32_t l1, l2, l3;
+};
+
+template <bool LANE_KEY>
+__device__ __forceinline__ void hut_block(uint32_t blk, uint32_t a, uint32_t h, uint32_t l, uint32_t k0, uint32_t k1,
+                                          uint32_t (&out)[4])
+{
+    blk = __builtin_amdgcn_readfirstlane(blk);
+    if (LANE_KEY) {
+        asm("" : "+v"(k0), "+v"(k1));
+    } else {
+        k0 = __builtin_amdgcn_readfirstlane(k0);
+        k1 = __builtin_amdgcn_readfirstlane(k1);
+        asm("" : "+s"(k0), "+s"(k1));
+    }
+    // rounds 1 and 2: after round 1 the counter is (X, a, s2, s3) with
+    // M0 X = (h, l)
+    const uint64_t b0 = (uint64_t)0xD2511F53u * blk;
+    const uint32_t s2 = (uint32_t)(b0 >> 32) ^ kHutTag ^ k1, s3 = (uint32_t)b0;
+    const uint64_t b1 = (uint64_t)0xCD9E8D57u * s2;
+    k0 += 0x9E3779B9u;
+    k1 += 0xBB67AE85u;
+    uint32_t c0 = (uint32_t)(b1 >> 32) ^ a ^ k0, c1 = (uint32_t)b1, c2 = h ^ s3 ^ k1, c3 = l;
+#pragma unroll
+    for (int r = 2; r < 10; ++r) {
+        k0 += 0x9E3779B9u;
+        k1 += 0xBB67AE85u;
+        const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
+        const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
+        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
+        const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        c1 = (uint32_t)p1;
+        c3 = (uint32_t)p0;
+        c0 = n0;
+        c2 = n2;
+    }
+    out[0] = c0; out[1] = c1; out[2] = c2; out[3] = c3;
+}
+
+// The next two pairs: from block blk, or with `odd` from the three words left
+// of the block before and the first of blk (the others are left).
+template <bool LANE_KEY>
+__device__ __attribute__((noinline)) HutPairs hut_pairs(uint32_t blk, uint32_t odd, uint32_t a, uint32_t h, uint32_t l,
+                                                        uint32_t k0, uint32_t k1, uint32_t l1, uint32_t l2, uint32_t l3)
+{
+    uint32_t w[4];
+    hut_block<LANE_KEY>(blk, a, h, l, k0, k1, w);
+    HutPairs r;
+    r.l1 = w[1];
+    r.l2 = w[2];
+    r.l3 = w[3];
+    if (__builtin_amdgcn_readfirstlane(odd)) {
+        w[3] = w[0];
+        w[0] = l1;
+        w[1] = l2;
+        w[2] = l3;
+    }
+    bm_pair(w[0], w[1], r.a0, r.b0);
+    bm_pair(w[2], w[3], r.a1, r.b1);
+    return r;
+}
+
 template <bool LANE_KEY>
 struct HutPhilox {
-    uint32_t k0, k1, e0, e1;
-    uint32_t pos;
-    uint32_t w[4];
+    uint32_t k0, k1, a, h, l;
+    uint32_t pos, blk;       // uniforms drawn; the next block
+    uint32_t odd, half;      // one uniform was drawn first; a pair is ready
+    uint32_t l1, l2, l3;
+    double ra, rb;
     template <uint32_t TAG>
     __device__ __forceinline__ void init_from(const PhiloxStreamT<TAG, LANE_KEY>& g)
     {
-        k0 = g.k0; k1 = g.k1; e0 = g.e0; e1 = g.e1;
-        pos = 0;
+        k0 = g.k0; k1 = g.k1;
+        const uint64_t p1 = (uint64_t)0xCD9E8D57u * g.e1;
+        const uint64_t p0 = (uint64_t)0xD2511F53u * ((uint32_t)(p1 >> 32) ^ g.e0 ^ g.k0);
+        a = (uint32_t)p1;
+        h = (uint32_t)(p0 >> 32);
+        l = (uint32_t)p0;
+        pos = 0; blk = 0; odd = 0; half = 0;
+        l1 = l2 = l3 = 0;
+        ra = rb = 0.0;
     }
+    // the one uniform, before any pair
     __device__ __forceinline__ double next()
     {
-        const uint32_t j = pos & 3u;
-        if (j == 0) philox4x32_10<LANE_KEY>(pos >> 2, e0, e1, kHutTag, k0, k1, w);
-        ++pos;
-        const uint32_t v = j == 0 ? w[0] : j == 1 ? w[1] : j == 2 ? w[2] : w[3];
-        return __builtin_fma((double)v, 0x1p-32, 0x1p-33);  // (v + 1/2) 2^-32, exact
+        uint32_t w[4];
+        hut_block<LANE_KEY>(0, a, h, l, k0, k1, w);
+        l1 = w[1]; l2 = w[2]; l3 = w[3];
+        pos = 1; blk = 1; odd = 1;
+        return __builtin_fma((double)w[0], 0x1p-32, 0x1p-33);  // (v + 1/2) 2^-32, exact
     }
-    __device__ __forceinline__ void gauss_pair(double& a, double& b)
+    __device__ __forceinline__ void gauss_pair(double& u, double& v)
     {
-        const double u1 = next();
-        const double u2 = next();
-        const double r = sqrt(-2.0 * bm_log(u1));
-        double sn, cs;
-        bm_sincos2pi(u2, sn, cs);
-        a = r * cs;
-        b = r * sn;
+        pos += 2;
+        if (half) {
+            u = ra;
+            v = rb;
+            half = 0;
+            return;
+        }
+        const HutPairs r = hut_pairs<LANE_KEY>(blk, odd, a, h, l, k0, k1, l1, l2, l3);
+        ++blk;
+        half = 1;
+        u = r.a0;
+        v = r.b0;
+        ra = r.a1;
+        rb = r.b1;
+        l1 = r.l1;
+        l2 = r.l2;
+        l3 = r.l3;
     }
     __device__ __forceinline__ uint32_t used() const { return pos; }
 };
@@ -428,17 +552,25 @@ __device__ __forceinline__ double theta_sigma(double m2, double p, double rad_le
 // value to a few units in the last place).
 struct ThetaCache {
     double p = -1.0, m2 = -1.0, a = 0.0, lb = 0.0;
+    __device__ __forceinline__ void set(const Track& t)
+    {
+        const double Es = 13.6;
+        p = t.p;
+        m2 = t.m2;
+        const double beta = p / sqrt(m2 + p * p);
+        a = Es / p / beta;
+        lb = log10(beta * beta);
+    }
+    // at the momentum of the last set()
+    __device__ __forceinline__ double at(double sqrt_rl, double log10_rl) const
+    {
+        const double epsilon = 0.088;
+        return a * sqrt_rl * (1.0 + epsilon * (log10_rl - lb));
+    }
     __device__ __forceinline__ double theta(const Track& t, double sqrt_rl, double log10_rl)
     {
-        const double Es = 13.6, epsilon = 0.088;
-        if (t.p != p || t.m2 != m2) {
-            p = t.p;
-            m2 = t.m2;
-            const double beta = p / sqrt(m2 + p * p);
-            a = Es / p / beta;
-            lb = log10(beta * beta);
-        }
-        return a * sqrt_rl * (1.0 + epsilon * (log10_rl - lb));
+        if (t.p != p || t.m2 != m2) set(t);
+        return at(sqrt_rl, log10_rl);
     }
 };
 

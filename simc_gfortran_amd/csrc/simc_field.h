@@ -9,6 +9,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "simc_device.h"
+
 namespace simcdev {
 
 constexpr int kTrgN = 51;                 // nz = nr = 51, trg_track.f:257-258
@@ -31,29 +33,6 @@ struct TrgMap {
     const TrgNode* node;
     double stht, ctht;
 };
-
-// Square root by one coupled (Goldschmidt) iteration from the hardware's
-// reciprocal square root (2^-24) and one residual correction (Markstein);
-// `y` receives 1 / sqrt(s) to 2^-47, enough for div_by's residual to round a
-// quotient.  Before their last rounding both results are within 2^-42 ulp;
-// for s in [2^-900, 2^1000] they equalled sqrt(s) and a / sqrt(s) on all of
-// 5e9 samples, without the scaling and special cases of the general forms.
-__device__ __forceinline__ double sqrt_inv(double s, double& y)
-{
-    const double y0 = __builtin_amdgcn_rsq(s);
-    double g = s * y0, h = 0.5 * y0;
-    const double e = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, e, g);
-    h = __builtin_fma(h, e, h);
-    y = h + h;
-    return __builtin_fma(__builtin_fma(-g, g, s), h, g);
-}
-// a / r from y = 1 / r to 2^-47
-__device__ __forceinline__ double div_by(double a, double r, double y)
-{
-    const double q = a * y;
-    return __builtin_fma(__builtin_fma(-r, q, a), y, q);
-}
 
 // trgField, trg_track.f:328-418.  The grid starts at 0 with spacing 2, so
 // zz(i) = 2 (i - 1), (z - zz(1)) / (zz(2) - zz(1)) = z / 2 exactly, and the

@@ -530,12 +530,28 @@ struct Hut {
     // parameter j of program step k, for the parameters that depend on the maps
     __device__ __forceinline__ double runtime_p(int k, int j) const { return ((coptr)a.ops)[k].p[j]; }
 
+    // Only a decay changes the momentum in the hut: the common variants form
+    // its factors once (run_hut) instead of comparing at every step.
+    __device__ __forceinline__ double theta(double sqrt_rl, double log10_rl)
+    {
+        if constexpr (RARE) return ms.theta(t, sqrt_rl, log10_rl);
+        else return ms.at(sqrt_rl, log10_rl);
+    }
+
     template <int CODE, int ARG, int STOP>
     __device__ __forceinline__ int step(int, double p0, double p1, double p2, double p3, double p4, double p5,
                                         double p6, double)
     {
         if constexpr (CODE == OP_PROJECT) {
-            project(g, t, F, p0);
+            if constexpr (RARE) {
+                project(g, t, F, p0);
+            } else {
+                // project without a decay; the root's argument is 1 or more
+                double y;
+                t.pathlen = t.pathlen + p0 * sqrt_inv(1.0 + t.dxdzs * t.dxdzs + t.dydzs * t.dydzs, y);
+                t.xs = t.xs + t.dxdzs * p0;
+                t.ys = t.ys + t.dydzs * p0;
+            }
         } else if constexpr (CODE == OP_RESMULT_DRAW) {
             resmult = hs.next() < p0 ? 2.0 : 1.0;
         } else if constexpr (CODE == OP_RESMULT_ONE) {
@@ -545,7 +561,7 @@ struct Hut {
             if (F.ms && p0 != 0.0) {
                 double d2, d3;
                 hs.gauss_pair(d2, d3);
-                const double ts = ms.theta(t, p1, p2);
+                const double ts = theta(p1, p2);
                 t.dydzs = t.dydzs + ts * d2;
                 t.dxdzs = t.dxdzs + ts * d3;
             }
@@ -555,12 +571,12 @@ struct Hut {
                 double d0, d1, d2, d3;
                 hs.gauss_pair(d0, d1);
                 hs.gauss_pair(d2, d3);
-                const double ts = ms.theta(t, p2, p3);
-                const double s12 = 3.4641016151377544;  // sqrt(12.)
+                const double ts = theta(p2, p3);
+                constexpr double s12 = 3.4641016151377544, r12 = 1.0 / s12;  // sqrt(12.)
                 t.dxdzs = t.dxdzs + ts * d0;
-                t.xs = t.xs + ts * p1 * d1 / s12 + ts * p1 * d0 / 2.0;
+                t.xs = t.xs + div_by(ts * p1 * d1, s12, r12) + ts * p1 * d0 / 2.0;
                 t.dydzs = t.dydzs + ts * d2;
-                t.ys = t.ys + ts * p1 * d3 / s12 + ts * p1 * d2 / 2.0;
+                t.ys = t.ys + div_by(ts * p1 * d3, s12, r12) + ts * p1 * d2 / 2.0;
             }
         } else if constexpr (CODE == OP_WIRE) {
             // plane STOP (0-based); a y plane when ARG = 1
@@ -626,11 +642,13 @@ __device__ __forceinline__ int run_hut(R& g, Track& t, const KArgs& a, const Fla
         S hs;
         hs.init_from(g);
         Hut<ARM, R, RARE, S> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ThetaCache{}, {0.0, 0.0, 0.0, 0.0}};
+        h.ms.set(t);
         const int st = hut_steps<ARM>(h);
         drawn = hs.used();
         return st;
     } else {
         Hut<ARM, R, RARE, R> h{g, g, t, a, F, off, lds_hits, resmult, 0, ThetaCache{}, {0.0, 0.0, 0.0, 0.0}};
+        h.ms.set(t);
         drawn = 0;
         return hut_steps<ARM>(h);
     }
