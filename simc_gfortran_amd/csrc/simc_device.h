@@ -64,6 +64,12 @@ constexpr uint32_t kPhiloxTag = 0x53494d43u;  // "SIMC"
 constexpr uint32_t kTargetTag = 0x54475453u;  // "TGTS"
 constexpr uint32_t kHutTag = 0x48555453u;     // "HUTS": the detector huts' draws
 
+// a ^ b ^ c in one instruction (truth table 0x96)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
 template <bool LANE_KEY = false>
 __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                               uint32_t k0, uint32_t k1, uint32_t out[4])
@@ -88,8 +94,8 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
     for (int r = 0; r < 10; ++r) {
         const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
         const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-        const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+        const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
         c1 = (uint32_t)p1;
         c3 = (uint32_t)p0;
         c0 = n0;
@@ -136,6 +142,20 @@ struct __attribute__((aligned(16))) BmLogEntry {
 static __constant__ BmLogEntry kBmLogTab[SIMC_BM_LOG_N] = SIMC_BM_LOG_TABLE;
 static __constant__ double kBmSinCosTab[SIMC_BM_SINCOS_N][2] = SIMC_BM_SINCOS_TABLE;
 
+// A 16-byte table entry at byte offset `off` from a table in constant memory:
+// one load from a scalar base and a 32-bit lane offset.
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 table16(const void* base, uint32_t off)
+{
+    typedef const char __attribute__((address_space(4)))* cbytes;
+    typedef const u32x4 __attribute__((address_space(4)))* centry;
+    return *(centry)((cbytes)base + off);
+}
+__device__ __forceinline__ double double_of(uint32_t lo, uint32_t hi)
+{
+    return __builtin_bit_cast(double, u32x2{lo, hi});
+}
+
 // Natural logarithm of u = (w + 1/2) 2^-32: u = m 2^e with m in [sqrt(1/2),
 // sqrt(2)), split on the bits (a 64-bit subtraction of sqrt(1/2)'s, whose
 // exponent field is then e); c = 1 + k/64 the nearest table point, k =
@@ -145,65 +165,97 @@ static __constant__ double kBmSinCosTab[SIMC_BM_SINCOS_N][2] = SIMC_BM_SINCOS_TA
 // to t^9 (truncation below 2^-56 relative); then e ln2 in two parts (ln2_hi
 // has 21 significant bits, so e ln2_hi is exact) and the table's two-part
 // -log(invc).
-__device__ __forceinline__ double bm_log(uint32_t w)
-{
-    const double u = __builtin_fma((double)w, 0x1p-32, 0x1p-33);  // exact
-    const uint64_t ub = __builtin_bit_cast(uint64_t, u);
-    const int e = (int)(uint32_t)((ub - 0x3fe6a09e667f3bcdull) >> 32) >> 20;
-    const uint32_t mhi = (uint32_t)(ub >> 32) - ((uint32_t)e << 20);
-    const double m = __builtin_bit_cast(double, ((uint64_t)mhi << 32) | (uint32_t)ub);
-    static_assert(SIMC_BM_LOG_K0 == 19, "the table's first point");
-    const double kd = __builtin_fma(m, 64.0, 0x1.8p52 - 64.0 + 20.0);  // low word: k + 20
-    const BmLogEntry L = kBmLogTab[(int)(uint32_t)__builtin_bit_cast(uint64_t, kd) - 1];
-    const double t = __builtin_fma(m, (double)L.invc, -1.0);
-    double q = 0x1.c71c71c71c71cp-4;                 // 1/9
-    q = __builtin_fma(t, q, -0x1p-3);                // -1/8
-    q = __builtin_fma(t, q, 0x1.2492492492492p-3);   // 1/7
-    q = __builtin_fma(t, q, -0x1.5555555555555p-3);  // -1/6
-    q = __builtin_fma(t, q, 0x1.999999999999ap-3);   // 1/5
-    q = __builtin_fma(t, q, -0x1p-2);                // -1/4
-    q = __builtin_fma(t, q, 0x1.5555555555555p-2);   // 1/3
-    q = __builtin_fma(t, q, -0x1p-1);                // -1/2
-    const double p = __builtin_fma(t * t, q, t);
-    const double de = (double)e;
-    return __builtin_fma(de, 0x1.62e42p-1, L.nhi + (p + __builtin_fma(de, 0x1.fdf473de6af28p-22, (double)L.nlo)));
-}
+struct BmLog {
+    double m;
+    int e;
+    u32x4 entry;
+    __device__ __forceinline__ void load(uint32_t w)
+    {
+        const u32x2 x = __builtin_bit_cast(u32x2, (double)w + 0.5);  // 2^32 u, exact
+        const uint32_t d = x.y - 0x3fe6a09eu - (x.x < 0x667f3bcdu ? 1u : 0u);
+        e = ((int)d >> 20) - 32;
+        m = double_of(x.x, x.y - (d & 0xfff00000u));
+        static_assert(SIMC_BM_LOG_K0 == 19, "the table's first point");
+        const double kd = __builtin_fma(m, 64.0, 0x1.8p52 - 64.0 + 20.0);  // low word: k + 20
+        entry = table16((const char*)kBmLogTab - 16, __builtin_bit_cast(u32x2, kd).x << 4);
+    }
+    __device__ __forceinline__ double value() const
+    {
+        const double nhi = double_of(entry.x, entry.y);
+        const float nlo = __builtin_bit_cast(float, (uint32_t)entry.z), invc = __builtin_bit_cast(float, (uint32_t)entry.w);
+        const double t = __builtin_fma(m, (double)invc, -1.0);
+        double q = 0x1.c71c71c71c71cp-4;                 // 1/9
+        q = __builtin_fma(t, q, -0x1p-3);                // -1/8
+        q = __builtin_fma(t, q, 0x1.2492492492492p-3);   // 1/7
+        q = __builtin_fma(t, q, -0x1.5555555555555p-3);  // -1/6
+        q = __builtin_fma(t, q, 0x1.999999999999ap-3);   // 1/5
+        q = __builtin_fma(t, q, -0x1p-2);                // -1/4
+        q = __builtin_fma(t, q, 0x1.5555555555555p-2);   // 1/3
+        q = __builtin_fma(t, q, -0x1p-1);                // -1/2
+        const double p = __builtin_fma(t * t, q, t);
+        const double de = (double)e;
+        return __builtin_fma(de, 0x1.62e42p-1, nhi + (p + __builtin_fma(de, 0x1.fdf473de6af28p-22, (double)nlo)));
+    }
+};
 
 // sin and cos of 2 pi u for u = (w + 1/2) 2^-32: 64 u = k + r with k =
 // rint(64 u) and r in [-1/2, 1/2], both read off w (its low 26 bits with
 // sign are 2^26 r - 1/2), d = r pi/32 in one fma; sin d and cos d by their
 // Taylor series to d^9 and d^8 (|d| <= pi/64, truncation below 2^-62), then
 // the rotation by the table's sin and cos of 2 pi k/64.
-__device__ __forceinline__ void bm_sincos2pi(uint32_t w, double& sn, double& cs)
-{
-    const uint32_t k = (w + (1u << 25)) >> 26;
-    const int rw = (int)(w << 6) >> 6;
-    const double d = __builtin_fma((double)rw, 0x1.921fb54442d18p-30, 0x1.921fb54442d18p-31);
-    const double z = d * d;
-    double ps = 0x1.71de3a556c734p-19;                 // 1/9!
-    ps = __builtin_fma(z, ps, -0x1.a01a01a01a01ap-13);  // -1/7!
-    ps = __builtin_fma(z, ps, 0x1.1111111111111p-7);    // 1/5!
-    ps = __builtin_fma(z, ps, -0x1.5555555555555p-3);   // -1/3!
-    const double sd = __builtin_fma(d * z, ps, d);
-    double pc = 0x1.a01a01a01a01ap-16;                 // 1/8!
-    pc = __builtin_fma(z, pc, -0x1.6c16c16c16c17p-10);  // -1/6!
-    pc = __builtin_fma(z, pc, 0x1.5555555555555p-5);    // 1/4!
-    pc = __builtin_fma(z, pc, -0x1p-1);                 // -1/2
-    const double cd = __builtin_fma(z, pc, 1.0);
-    const double sa = kBmSinCosTab[k][0], ca = kBmSinCosTab[k][1];
-    sn = __builtin_fma(sa, cd, ca * sd);
-    cs = __builtin_fma(ca, cd, -(sa * sd));
-}
+struct BmSinCos {
+    uint32_t w;
+    u32x4 entry;
+    __device__ __forceinline__ void load(uint32_t w_)
+    {
+        w = w_;
+        entry = table16(kBmSinCosTab, ((w + (1u << 25)) >> 22) & 0x3f0u);  // entry k
+    }
+    __device__ __forceinline__ void value(double& sn, double& cs) const
+    {
+        const int rw = (int)(w << 6) >> 6;
+        const double d = __builtin_fma((double)rw, 0x1.921fb54442d18p-30, 0x1.921fb54442d18p-31);
+        const double z = d * d;
+        double ps = 0x1.71de3a556c734p-19;                 // 1/9!
+        ps = __builtin_fma(z, ps, -0x1.a01a01a01a01ap-13);  // -1/7!
+        ps = __builtin_fma(z, ps, 0x1.1111111111111p-7);    // 1/5!
+        ps = __builtin_fma(z, ps, -0x1.5555555555555p-3);   // -1/3!
+        const double sd = __builtin_fma(d * z, ps, d);
+        double pc = 0x1.a01a01a01a01ap-16;                 // 1/8!
+        pc = __builtin_fma(z, pc, -0x1.6c16c16c16c17p-10);  // -1/6!
+        pc = __builtin_fma(z, pc, 0x1.5555555555555p-5);    // 1/4!
+        pc = __builtin_fma(z, pc, -0x1p-1);                 // -1/2
+        const double cd = __builtin_fma(z, pc, 1.0);
+        const double sa = double_of(entry.x, entry.y), ca = double_of(entry.z, entry.w);
+        sn = __builtin_fma(sa, cd, ca * sd);
+        cs = __builtin_fma(ca, cd, -(sa * sd));
+    }
+};
 
 // The Box-Muller pair of two words: sqrt(-2 ln u1) (cos 2 pi u2, sin 2 pi u2).
 // -2 ln u1 lies in [2^-32, 46], inside sqrt_inv's range.
-__device__ __forceinline__ void bm_pair(uint32_t w1, uint32_t w2, double& c, double& sn_)
+struct BmPair {
+    BmLog lg;
+    BmSinCos sc;
+    __device__ __forceinline__ void load(uint32_t w1, uint32_t w2)
+    {
+        lg.load(w1);
+        sc.load(w2);
+    }
+    __device__ __forceinline__ void value(double& c, double& s) const
+    {
+        double y, sn, cs;
+        const double r = sqrt_inv(-2.0 * lg.value(), y);
+        sc.value(sn, cs);
+        c = r * cs;
+        s = r * sn;
+    }
+};
+__device__ __forceinline__ void bm_pair(uint32_t w1, uint32_t w2, double& c, double& s)
 {
-    double y, sn, cs;
-    const double r = sqrt_inv(-2.0 * bm_log(w1), y);
-    bm_sincos2pi(w2, sn, cs);
-    c = r * cs;
-    sn_ = r * sn;
+    BmPair p;
+    p.load(w1, w2);
+    p.value(c, s);
 }
 
 // TAG is the fourth counter word: streams of different tags are independent
@@ -351,8 +403,8 @@ __device__ __forceinline__ void hut_block(uint32_t blk, uint32_t a, uint32_t h, 
         k1 += 0xBB67AE85u;
         const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
         const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-        const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+        const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+        const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
         c1 = (uint32_t)p1;
         c3 = (uint32_t)p0;
         c0 = n0;
@@ -379,8 +431,13 @@ __device__ __attribute__((noinline)) HutPairs hut_pairs(uint32_t blk, uint32_t o
         w[1] = l2;
         w[2] = l3;
     }
-    bm_pair(w[0], w[1], r.a0, r.b0);
-    bm_pair(w[2], w[3], r.a1, r.b1);
+    // all four table reads in flight before the first is waited for
+    BmPair p0, p1;
+    p0.load(w[0], w[1]);
+    p1.load(w[2], w[3]);
+    __builtin_amdgcn_sched_barrier(0);
+    p0.value(r.a0, r.b0);
+    p1.value(r.a1, r.b1);
     return r;
 }
 
