@@ -833,41 +833,39 @@ __device__ __forceinline__ void rotate_vaxis(const Track& t, const Rot& r, doubl
     xp0 = xp0 + yi * beta_p * r.sin_th;
 }
 
-// enerloss_new, enerloss_new.f:19-82
+// enerloss_new, enerloss_new.f:19-82, typeflag 1, in the collimator's
+// tungsten: dens = 17, Z = 69.45, A = 171.56797.  Its material terms (the
+// mean excitation I = 16 Z^0.9 eV, the plasma energy hnup, CO = ln hnup -
+// ln I + 1/2, ln(me/I^2) + 1.063) are literals, each the correctly rounded
+// value of the reference's expression; only the logarithms of the particle's
+// terms are left to each step.
 template <class R>
-__device__ double enerloss_new(R& g, double len, double dens, double zeff, double aeff,
-                               double epart, double mpart, int typeflag)
+__device__ double enerloss_tungsten(R& g, double len, double epart, double mpart)
 {
-    const double me = 0.51099906;
+    const double dens = 17.0, zeff = 69.45, aeff = 171.56797;
+    const double CO = -0x1.c387569315210p+0, ln10 = 0x1.26bb1bbb55516p+1, ln_me_I2 = 0x1.db05066e9762dp+3;
     const double thick = len * dens;
     const double gamma = epart / mpart;
     const double beta = sqrt(1.0 - 1.0 / (gamma * gamma));
-    const double I = zeff == 1.0 ? 21.8e-06 : (16.0 * pow(zeff, 0.9)) * 1.0e-06;
-    const double hnup = 28.816e-06 * sqrt(dens * zeff / aeff);
-    const double log10bg = log(beta * gamma) / log(10.0);
-    const double CO = log(hnup) - log(I) + 0.5;
+    const double lnbg = log(beta * gamma);
+    const double log10bg = lnbg / ln10;
     double denscorr;
     if (log10bg < 0.0) denscorr = 0.0;
     else if (log10bg < 3.0) {
         const double t3 = 3.0 - log10bg;
-        denscorr = CO + log(10.0) * log10bg + fabs(CO / 27.0) * (t3 * t3 * t3);
-    } else if (log10bg < 4.7) denscorr = CO + log(10.0) * log10bg;
-    else denscorr = CO + log(10.0) * 4.7;
+        denscorr = CO + ln10 * log10bg + fabs(CO / 27.0) * (t3 * t3 * t3);
+    } else if (log10bg < 4.7) denscorr = CO + ln10 * log10bg;
+    else denscorr = CO + ln10 * 4.7;
     double E;
     if (thick <= 0.0) {
         E = 0.0;
     } else {
         const double b2 = beta * beta;
         const double mp_new = 0.1536e-03 * zeff / aeff * thick / b2 *
-                              (log(me / (I * I)) + 1.063 + 2.0 * log(gamma * beta) +
-                               log(0.1536 * zeff / aeff * thick / b2) - b2 - denscorr);
+                              (ln_me_I2 + 2.0 * lnbg + log(0.1536 * zeff / aeff * thick / b2) - b2 - denscorr);
         const double mp = mp_new * 1000.0;
         const double chsi = 0.307075 / 2.0 * zeff / aeff * thick / b2;
-        double x = 0.0;
-        if (typeflag == 1) x = fabs(gauss1(g, 10.0));
-        else if (typeflag == 2) x = 3.0;
-        else if (typeflag == 3) x = 0.0067;
-        else if (typeflag == 4) x = 1.0;
+        const double x = fabs(gauss1(g, 10.0));
         const double lambda = x > 0.0 ? -2.0 * log(x) : 100000.0;
         E = lambda * chsi + mp;
     }
@@ -888,30 +886,36 @@ __device__ __forceinline__ double times_1em27_quad(double a)
     return p + (e + a * lo);
 }
 
-// pion_coll_absorb, hms/pion_coll_absorb.f:54-90: transmission probability
-__device__ double pion_coll_absorb(double ppi, double thick)
+// pion_coll_absorb, hms/pion_coll_absorb.f:54-90: transmission probability.
+// The pion-nucleus cross sections sigreac * 171.57^qreac are taken per energy
+// from a table (correctly rounded powers); the interval is found by counting
+// the energies below the pion's, the same instructions in every lane.
+struct __attribute__((aligned(16))) PionSigma {
+    double T, sig;
+};
+static __constant__ PionSigma kPionSigma[14] = {
+    {85.0, 0x1.ab340a64878aep+11},    {125.0, 0x1.3968509ef4563p+11},   {165.0, 0x1.05839ee881132p+11},
+    {205.0, 0x1.ca66f5587393fp+10},   {245.0, 0x1.a50c4a4680271p+10},   {315.0, 0x1.8d13de1ddb713p+10},
+    {584.02, 0x1.837068a094a21p+10},  {711.95, 0x1.830f350eff357p+10},  {870.12, 0x1.89f7ddd21c59dp+10},
+    {1227.57, 0x1.8667eaf51ddc9p+10}, {1446.58, 0x1.85616242b8899p+10}, {1865.29, 0x1.7268c936690eep+10},
+    {2858.0, 0x1.9f2eb6e68240ap+10},  {4159.0, 0x1.b493a5d2fff03p+10}};
+
+__device__ __forceinline__ double pion_coll_absorb(double ppi, double thick)
 {
-    const double T[14] = {85.0, 125.0, 165.0, 205.0, 245.0, 315.0, 584.02, 711.95, 870.12,
-                          1227.57, 1446.58, 1865.29, 2858.0, 4159.0};
-    const double sigreac[14] = {26.03, 84.47, 117.3, 117.4, 101.9, 69.58, 42.5, 44.7, 47.9,
-                                46.5, 45.2, 39.6, 35.34, 33.15};
-    const double qreac[14] = {0.948, 0.659, 0.56, 0.5342, 0.5452, 0.60796, 0.699, 0.689,
-                              0.679, 0.683, 0.688, 0.704, 0.7483, 0.7705};
     const double Navagadro = 6.0221367e+23, mpi = 139.56995;
     const double mate_dens = 17.0, mate_A = 171.57;
     const double Epi = sqrt(ppi * ppi + mpi * mpi);
     const double Tpi = Epi - mpi;
+    int below = 0;
+#pragma unroll
+    for (int i = 0; i < 14; ++i) below += Tpi > kPionSigma[i].T ? 1 : 0;
     double sigA = 0.0;
-    for (int i = 0; i < 13; ++i) {
-        if (Tpi > T[i] && Tpi <= T[i + 1]) {
-            const double Thi = T[i + 1], Tlo = T[i];
-            const double sigAhi = sigreac[i + 1] * pow(mate_A, qreac[i + 1]);
-            const double sigAlo = sigreac[i] * pow(mate_A, qreac[i]);
-            sigA = (sigAlo * (Thi - Tpi) + sigAhi * (Tpi - Tlo)) / (Thi - Tlo);
-            sigA = times_1em27_quad(sigA);
-        }
+    if (below == 14) {
+        sigA = times_1em27_quad(kPionSigma[13].sig);
+    } else if (below > 0) {
+        const PionSigma lo = kPionSigma[below - 1], hi = kPionSigma[below];
+        sigA = times_1em27_quad((lo.sig * (hi.T - Tpi) + hi.sig * (Tpi - lo.T)) / (hi.T - lo.T));
     }
-    if (Tpi > T[13]) sigA = times_1em27_quad(sigreac[13] * pow(mate_A, qreac[13]));
     const double lambdai = mate_dens * Navagadro * sigA / mate_A;
     return exp(-(0.0 + thick * lambdai));
 }
@@ -926,10 +930,10 @@ template <class R>
 __device__ bool coll_step(R& g, Track& t, const Flags& F, const CollGeom& G, double p_spec,
                           unsigned* cnt_step)
 {
-    const double coll_dens = 17.0, zcoll = 69.45, acoll = 171.56797;
     const int nstep = 20;
     double h_step = G.h_entr, v_step = G.v_entr;
     double epart = sqrt(t.p * t.p + t.m2);
+#pragma unroll 1
     for (int n = 1; n <= nstep; ++n) {
         bool step_flag = false;
         if (fabs(t.ys - G.y_off) > h_step) { step_flag = true; ++cnt_step[0]; }
@@ -946,7 +950,7 @@ __device__ bool coll_step(R& g, Track& t, const Flags& F, const CollGeom& G, dou
             }
             musc(g, t, thick / G.coll_radl, t.dydzs, t.dxdzs);
             epart = sqrt(t.p * t.p + t.m2);
-            const double eloss = enerloss_new(g, thick, coll_dens, zcoll, acoll, epart, sqrt(t.m2), 1);
+            const double eloss = enerloss_tungsten(g, thick, epart, sqrt(t.m2));
             epart = epart - eloss;
             if (epart < sqrt(t.m2)) return false;
             t.p = sqrt(epart * epart - t.m2);

@@ -366,7 +366,13 @@ __device__ __forceinline__ void fit_track(const Flags& F, const double* lds, con
 // run-time polynomial tables (a copy of its own, so that the compiled
 // polynomials' code is not shaped by the other path).
 // ---------------------------------------------------------------------------
-template <int ARM, class R, bool RARE, bool GEN>
+// Only the SHMS has a COSY segment (its bender) ahead of the collimator: the
+// other arms' first stage holds no polynomial (TRANSP false; load_arm checks
+// their programs), and its kernels no polynomial's registers.
+template <int ARM>
+constexpr bool kTranspBeforeCollimator = ARM == SIMC_ARM_SHMS;
+
+template <int ARM, class R, bool RARE, bool GEN, bool TRANSP>
 __device__ __forceinline__ int run_program(R& g, Track& t, const KArgs& a, const Flags& FA, uint32_t off,
                                            unsigned* coll_cnt, int pc_begin, int pc_end)
 {
@@ -391,20 +397,23 @@ __device__ __forceinline__ int run_program(R& g, Track& t, const KArgs& a, const
         case OP_PROJECT:
             project(g, t, F, p0);
             break;
-        case OP_TRANSP: {
-            const int cls = ops[pc].arg;
-            transp(g, t, F, p0, [&](double r0, double r1, double r2, double r3, double r4, double& o0,
-                                    double& o1, double& o2, double& o3, double& o4) {
-                if constexpr (GEN) {
-                    double o[5];
-                    poly_generic<5>((cuptr)a.gen, cls, r0, r1, r2, r3, r4, o);
-                    o0 = o[0]; o1 = o[1]; o2 = o[2]; o3 = o[3]; o4 = o[4];
-                } else {
-                    poly_fwd<ARM>(cls, coef, r0, r1, r2, r3, r4, o0, o1, o2, o3, o4);
-                }
-            });
+        case OP_TRANSP:
+            if constexpr (TRANSP) {
+                const int cls = ops[pc].arg;
+                transp(g, t, F, p0, [&](double r0, double r1, double r2, double r3, double r4, double& o0,
+                                        double& o1, double& o2, double& o3, double& o4) {
+                    if constexpr (GEN) {
+                        double o[5];
+                        poly_generic<5>((cuptr)a.gen, cls, r0, r1, r2, r3, r4, o);
+                        o0 = o[0]; o1 = o[1]; o2 = o[2]; o3 = o[3]; o4 = o[4];
+                    } else {
+                        poly_fwd<ARM>(cls, coef, r0, r1, r2, r3, r4, o0, o1, o2, o3, o4);
+                    }
+                });
+            } else {
+                st = ST_BADOP;
+            }
             break;
-        }
         case OP_CHECK_R2:
             if ((t.xs * t.xs + t.ys * t.ys) > p0) st = ops[pc].stop;
             break;
@@ -497,7 +506,8 @@ __device__ __forceinline__ int run_program(R& g, Track& t, const KArgs& a, const
 }
 
 // ---------------------------------------------------------------------------
-// The detector hut, compiled.  gen_hut.cpp writes the hut steps of each arm
+// The detector hut, compiled (and interpreted where hut_path says so).
+// gen_hut.cpp writes the hut steps of each arm
 // family as straight-line code (hut_gen.inc): one step<code, arg, stop>(k,
 // p0..p7) call per step k of the program, its parameters as literals where
 // they do not depend on the loaded maps.  The library checks every loaded
@@ -510,10 +520,7 @@ __device__ __forceinline__ int run_program(R& g, Track& t, const KArgs& a, const
 // stream hs (HutStreamOf); in-flight decays in the drifts draw from the arm's
 // stream g.  Wire hits go to LDS (hits[plane][lane]).
 // ---------------------------------------------------------------------------
-template <int>
-constexpr bool kNotHutStep = false;
-
-template <int ARM, class R, bool RARE, class S>
+template <int ARM, class R, bool RARE, class S, bool GENERAL>
 struct Hut {
     R& g;
     S& hs;
@@ -538,12 +545,22 @@ struct Hut {
         else return ms.at(sqrt_rl, log10_rl);
     }
 
+    // Step k of the compiled program: its code, argument and stop code are literals.
     template <int CODE, int ARG, int STOP>
     __device__ __forceinline__ int step(int, double p0, double p1, double p2, double p3, double p4, double p5,
                                         double p6, double)
     {
-        if constexpr (CODE == OP_PROJECT) {
-            if constexpr (RARE) {
+        static_assert(CODE == OP_PROJECT || (CODE >= OP_RESMULT_DRAW && CODE <= OP_FIDUCIAL) || CODE == OP_BOX_ROT_H,
+                      "not a detector-hut step");
+        return run(CODE, ARG, STOP, p0, p1, p2, p3, p4, p5, p6);
+    }
+
+    __device__ __forceinline__ int run(int code, int arg, int stop, double p0, double p1, double p2, double p3,
+                                       double p4, double p5, double p6)
+    {
+        switch (code) {
+        case OP_PROJECT:
+            if constexpr (GENERAL) {
                 project(g, t, F, p0);
             } else {
                 // project without a decay; the root's argument is 1 or more
@@ -552,11 +569,14 @@ struct Hut {
                 t.xs = t.xs + t.dxdzs * p0;
                 t.ys = t.ys + t.dydzs * p0;
             }
-        } else if constexpr (CODE == OP_RESMULT_DRAW) {
+            break;
+        case OP_RESMULT_DRAW:
             resmult = hs.next() < p0 ? 2.0 : 1.0;
-        } else if constexpr (CODE == OP_RESMULT_ONE) {
+            break;
+        case OP_RESMULT_ONE:
             resmult = 1.0;
-        } else if constexpr (CODE == OP_MUSC) {
+            break;
+        case OP_MUSC:
             // musc(m2,p,radw,dydzs,dxdzs): first draw to y', second to x'
             if (F.ms && p0 != 0.0) {
                 double d2, d3;
@@ -565,7 +585,8 @@ struct Hut {
                 t.dydzs = t.dydzs + ts * d2;
                 t.dxdzs = t.dxdzs + ts * d3;
             }
-        } else if constexpr (CODE == OP_MUSC_EXT) {
+            break;
+        case OP_MUSC_EXT:
             // musc_ext(...,dydzs,dxdzs,ys,xs): (x', x) then (y', y)
             if (F.ms && p0 != 0.0 && p1 > 0.0 && p0 >= 0.0) {
                 double d0, d1, d2, d3;
@@ -573,24 +594,31 @@ struct Hut {
                 hs.gauss_pair(d2, d3);
                 const double ts = theta(p2, p3);
                 constexpr double s12 = 3.4641016151377544, r12 = 1.0 / s12;  // sqrt(12.)
+                const double ax = ts * p1 * d1, ay = ts * p1 * d3;
                 t.dxdzs = t.dxdzs + ts * d0;
-                t.xs = t.xs + div_by(ts * p1 * d1, s12, r12) + ts * p1 * d0 / 2.0;
+                t.xs = t.xs + (GENERAL ? ax / s12 : div_by(ax, s12, r12)) + ts * p1 * d0 / 2.0;
                 t.dydzs = t.dydzs + ts * d2;
-                t.ys = t.ys + div_by(ts * p1 * d3, s12, r12) + ts * p1 * d2 / 2.0;
+                t.ys = t.ys + (GENERAL ? ay / s12 : div_by(ay, s12, r12)) + ts * p1 * d2 / 2.0;
             }
-        } else if constexpr (CODE == OP_WIRE) {
-            // plane STOP (0-based); a y plane when ARG = 1
+            break;
+        case OP_WIRE: {
+            // plane `stop` (0-based); a y plane when arg = 1
             double d2 = 0.0, d3 = 0.0;
             if (F.wcs) hs.gauss_pair(d2, d3);
-            const double h = ARG ? t.ys + F.sigma * d3 * resmult : t.xs + F.sigma * d2 * resmult;
-            lds_hits[STOP * kBlock + threadIdx.x] = h;
-        } else if constexpr (CODE == OP_BOX) {
-            if (t.xs > p0 || t.xs < p1 || t.ys > p2 || t.ys < p3) return STOP;
-        } else if constexpr (CODE == OP_SCIN) {
+            const double h = arg ? t.ys + F.sigma * d3 * resmult : t.xs + F.sigma * d2 * resmult;
+            lds_hits[stop * kBlock + threadIdx.x] = h;
+            break;
+        }
+        case OP_BOX:
+            if (t.xs > p0 || t.xs < p1 || t.ys > p2 || t.ys < p3) return stop;
+            break;
+        case OP_SCIN:
             if (t.ys < p0 && t.ys > p1 && t.xs < p2 && t.xs > p3) ++scincount;
-        } else if constexpr (CODE == OP_TRIGGER) {
-            if (scincount < ARG) return STOP;
-        } else if constexpr (CODE == OP_FIT) {
+            break;
+        case OP_TRIGGER:
+            if (scincount < arg) return stop;
+            break;
+        case OP_FIT: {
             const ctptr tab = (ctptr)a.tab;
             double zdc[12];
 #pragma unroll
@@ -600,20 +628,39 @@ struct Hut {
             st64(a.dx_fp, a.n_arr, off, fp[1]);
             st64(a.y_fp, a.n_arr, off, fp[2]);
             st64(a.dy_fp, a.n_arr, off, fp[3]);
-        } else if constexpr (CODE == OP_BOX_ROT_H) {
+            break;
+        }
+        case OP_BOX_ROT_H: {
             const Rot r{p0, p1, p2};
             double xr = t.xs, yr = t.ys;
             rotate_haxis(t, r, xr, yr);
-            if (xr > p3 || xr < p4 || yr > p5 || yr < p6) return STOP;
-        } else if constexpr (CODE == OP_FIDUCIAL) {
+            if (xr > p3 || xr < p4 || yr > p5 || yr < p6) return stop;
+            break;
+        }
+        case OP_FIDUCIAL: {
             // track of the fit at z = p0
             const double xcal = fp[0] + fp[1] * p0;
             const double ycal = fp[2] + fp[3] * p0;
-            if (ycal > p1 || ycal < p2 || xcal > p3 || xcal < p4) return STOP;
-        } else {
-            static_assert(kNotHutStep<CODE>, "not a detector-hut step");
+            if (ycal > p1 || ycal < p2 || xcal > p3 || xcal < p4) return stop;
+            break;
+        }
+        default:
+            return ST_BADOP;  // not a hut step (excluded by the host's check)
         }
         return ST_OK;
+    }
+
+    // The program's steps from pc on, interpreted: one copy of each step's code.
+    __device__ __forceinline__ int loop(int pc)
+    {
+        const coptr ops = (coptr)a.ops;
+        for (;; ++pc) {
+            const coptr o = ops + pc;
+            const int code = o->code;
+            if (code == OP_END) return ST_OK;
+            const int st = run(code, o->arg, o->stop, o->p[0], o->p[1], o->p[2], o->p[3], o->p[4], o->p[5], o->p[6]);
+            if (st) return st;
+        }
     }
 };
 
@@ -626,11 +673,37 @@ __device__ __forceinline__ int hut_steps(H& h)
     else return hut_steps_hrs(h);
 }
 
-// One event through its arm's compiled hut: ST_OK or the stop code; `drawn`
-// receives the uniforms taken from the hut's own stream.
+// The compiled steps, or the interpreted ones.  The common variants run the
+// compiled steps, whose drifts and thick layers take roots and quotients
+// without the special cases of the general forms; a wavefront with an event
+// that could meet those (slopes or a scattering angle beyond any track's, or
+// not numbers) is interpreted in the general form.  The RARE variants, whose
+// drifts hold the decay, are always interpreted: with a copy of it at each of
+// 60 drifts they were 330 KB of code (HMS pions with decay, 1e6: 0.58 -> 0.53
+// ms; the common hut interpreted takes 2.19 ms for SHMS 1e7, compiled 1.50:
+// it waits for the step records' scalar loads).
+template <int ARM, class R, bool RARE, class S>
+__device__ __forceinline__ int hut_path(R& g, S& hs, Track& t, const KArgs& a, const Flags& F, uint32_t off,
+                                        double* lds_hits, double& resmult, int pc)
+{
+    ThetaCache ms;
+    ms.set(t);
+    if constexpr (!RARE) {
+        const bool plain = fabs(t.dxdzs) < 1.e6 && fabs(t.dydzs) < 1.e6 && ms.a < 1.e6 && fabs(ms.lb) < 1.e6;
+        if (__all(plain)) {
+            Hut<ARM, R, RARE, S, false> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ms, {0.0, 0.0, 0.0, 0.0}};
+            return hut_steps<ARM>(h);
+        }
+    }
+    Hut<ARM, R, RARE, S, true> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ms, {0.0, 0.0, 0.0, 0.0}};
+    return h.loop(pc);
+}
+
+// One event through its arm's hut: ST_OK or the stop code; `drawn` receives
+// the uniforms taken from the hut's own stream.
 template <int ARM, class R, bool RARE>
 __device__ __forceinline__ int run_hut(R& g, Track& t, const KArgs& a, const Flags& FA, uint32_t off,
-                                       double* lds_hits, double& resmult, uint32_t& drawn)
+                                       double* lds_hits, double& resmult, uint32_t& drawn, int pc)
 {
     Flags F = FA;
     if (!RARE) {  // in-flight decay only in the RARE variant (as in the magnets)
@@ -641,16 +714,12 @@ __device__ __forceinline__ int run_hut(R& g, Track& t, const KArgs& a, const Fla
     if constexpr (HutStreamOf<R>::kOwn) {
         S hs;
         hs.init_from(g);
-        Hut<ARM, R, RARE, S> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ThetaCache{}, {0.0, 0.0, 0.0, 0.0}};
-        h.ms.set(t);
-        const int st = hut_steps<ARM>(h);
+        const int st = hut_path<ARM, R, RARE, S>(g, hs, t, a, F, off, lds_hits, resmult, pc);
         drawn = hs.used();
         return st;
     } else {
-        Hut<ARM, R, RARE, R> h{g, g, t, a, F, off, lds_hits, resmult, 0, ThetaCache{}, {0.0, 0.0, 0.0, 0.0}};
-        h.ms.set(t);
         drawn = 0;
-        return hut_steps<ARM>(h);
+        return hut_path<ARM, R, RARE, R>(g, g, t, a, F, off, lds_hits, resmult, pc);
     }
 }
 
@@ -812,10 +881,11 @@ __device__ __forceinline__ void count_slit(const KArgs& a, unsigned* hist, uint3
 // the hut stage, TO_Q lists the accepted events (index and setting) for
 // recon_list_kernel instead of reconstructing them here.
 // The common variants are held to three wavefronts per SIMD (168 VGPRs),
-// the hut stage to four (128 VGPRs: a few values spill to scratch, and the
-// extra wavefront hides more of the hut's latency than the spills cost), the
-// RARE variants to two (256 VGPRs, a few spills; at one wavefront a pion run
-// with decay took 1.45 x as long).
+// the hut stage to four (128 VGPRs: a few values may spill to scratch, and
+// the extra wavefront hides more of the hut's latency than the spills cost),
+// the RARE variants to two (256 VGPRs, a few spills; at one wavefront a pion
+// run with decay took 1.45 x as long, at three the spills cost more than the
+// wavefront gives).
 template <int ARM, class R, bool RARE, int STAGE, bool FROM_Q, bool TO_Q>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2 : (STAGE == STAGE_HUT ? 4 : 3)))) void stage_kernel(
     KArgs a, Queue qin, Queue qout, int32_t pc_begin, int32_t pc_end)
@@ -901,9 +971,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2
         }
         int st;
         uint32_t hut_drawn = 0;
-        if constexpr (STAGE == STAGE_HUT) st = run_hut<ARM, R, RARE>(g, t, a, F, e.off, lds_hits, resmult, hut_drawn);
-        else if (a.gen) st = run_program<ARM, R, RARE, true>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
-        else st = run_program<ARM, R, RARE, false>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
+        if constexpr (STAGE == STAGE_HUT) st = run_hut<ARM, R, RARE>(g, t, a, F, e.off, lds_hits, resmult, hut_drawn, pc_begin);
+        else if constexpr (!FROM_Q && !kTranspBeforeCollimator<ARM>)
+            st = run_program<ARM, R, RARE, false, false>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
+        else if (a.gen) st = run_program<ARM, R, RARE, true, true>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
+        else st = run_program<ARM, R, RARE, false, true>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
         const uint32_t used = (uint32_t)g.used() + hut_drawn;
         if (g.overflow) st = ST_TAPE;
         if (STAGE == STAGE_HUT) {
@@ -2179,6 +2251,9 @@ int load_arm(simc_ctx* ctx, int arm, const std::string& fwd_path, const std::str
         if (first == 0 || first == hut) return fail(SIMC_E_INTERNAL, "no stage split before the hut");
         ctx->coll_pc[ai] = first;
     }
+    if (arm != SIMC_ARM_SHMS)   // kTranspBeforeCollimator
+        for (int k = 0; k < ctx->coll_pc[ai]; ++k)
+            if (P.ops[k].code == OP_TRANSP) return fail(SIMC_E_INTERNAL, "a COSY segment before the collimator");
     HIPCHK(hipMalloc(&ctx->d_coef[ai], packed.size() * sizeof(double)));
     HIPCHK(hipMemcpy(ctx->d_coef[ai], packed.data(), packed.size() * sizeof(double), hipMemcpyHostToDevice));
     if (!gen_bytes.empty()) {
