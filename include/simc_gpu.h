@@ -164,6 +164,15 @@ int simc_hrsl_run(simc_ctx *ctx, const simc_settings *s, const simc_events_in *i
 int simc_arm_run(simc_ctx *ctx, int arm, const simc_settings *s, const simc_events_in *in,
                  simc_events_out *out, int64_t n, const simc_rng *rng, void *stream);
 
+/* simc_arm_run into outputs that hold nothing yet (no counterpart in the
+ * reference): the INOUT columns pathlen, resmult and x_fp..dy_fp start from 0
+ * instead of their contents, and every given column is written for every
+ * event, so that the caller neither clears nor copies anything first.  The
+ * outputs must not alias the inputs' dxdz, dydz, dpp, y.  Not with the mock
+ * sieve (SIMC_E_ARG), whose forced angles are INOUT. */
+int simc_arm_run_fresh(simc_ctx *ctx, int arm, const simc_settings *s, const simc_events_in *in,
+                       simc_events_out *out, int64_t n, const simc_rng *rng, void *stream);
+
 /* simc_arm_run without any allocation (no counterpart in the reference: for
  * callers that cannot allocate device memory, such as code under HIP graph
  * capture or a tight serving loop).  The survivor queues live in a static
@@ -190,6 +199,10 @@ int simc_arm_run_noalloc(simc_ctx *ctx, int arm, const simc_settings *s, const s
  * montecarlo() (simc.f:1464-1488).  Calls on one context are serialised. */
 int simc_arm_run_host(simc_ctx *ctx, int arm, const simc_settings *s, const simc_events_in *in,
                       simc_events_out *out, int64_t n, const simc_rng *rng);
+/* The same for outputs that hold nothing yet (see simc_arm_run_fresh): only
+ * the inputs are sent. */
+int simc_arm_run_host_fresh(simc_ctx *ctx, int arm, const simc_settings *s, const simc_events_in *in,
+                            simc_events_out *out, int64_t n, const simc_rng *rng);
 
 /* simc_recon_run on host arrays (synchronous, as simc_arm_run_host). */
 int simc_recon_run_host(simc_ctx *ctx, int arm, int64_t n, const double *x_fp, const double *dx_fp,
@@ -241,6 +254,10 @@ int simc_batch_create(simc_ctx *ctx, const simc_setting *settings, int n_setting
 /* in / out: device arrays covering every setting's range (the plain run's
  * semantics per event). */
 int simc_batch_run(simc_batch *b, const simc_events_in *in, simc_events_out *out, void *stream);
+
+/* The same for outputs that hold nothing yet (see simc_arm_run_fresh);
+ * elements outside every setting's range are not written. */
+int simc_batch_run_fresh(simc_batch *b, const simc_events_in *in, simc_events_out *out, void *stream);
 /* STOP counters of setting i (input order) from the last run, common-block order. */
 int simc_batch_counters(simc_batch *b, int setting, int64_t *c, int ncounters);
 /* Launch tile: events per launch sequence (256 .. 2^24; reserves queues). */

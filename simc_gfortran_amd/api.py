@@ -62,6 +62,7 @@ COUNTERS = {HMS: HMS_COUNTERS, SOS: SOS_COUNTERS, HRSR: HRS_COUNTERS, HRSL: HRS_
 EXPORTS = [
     "simc_ctx_create", "simc_ctx_create_files", "simc_ctx_load_arm", "simc_ctx_destroy",
     "simc_hms_run", "simc_shms_run", "simc_sos_run", "simc_hrsr_run", "simc_hrsl_run", "simc_arm_run",
+    "simc_arm_run_fresh", "simc_arm_run_host_fresh", "simc_batch_run_fresh",
     "simc_arm_run_noalloc", "simc_arm_run_timed", "simc_recon_run", "simc_counters_get",
     "simc_counters_reset", "simc_map_class_info", "simc_poly_flops_full", "simc_stop_flops",
     "simc_stop_flops_stage", "simc_stop_flops_hut", "simc_arm_run_host", "simc_recon_run_host",
@@ -237,12 +238,14 @@ def library(path: str = LIB_PATH):
                                C.POINTER(EventsOut), C.c_int64, C.POINTER(Rng), _vp]
     L.simc_arm_run_noalloc.argtypes = [_vp, C.c_int, C.POINTER(Settings), C.POINTER(EventsIn),
                                        C.POINTER(EventsOut), C.c_int64, C.POINTER(Rng), _vp]
+    L.simc_arm_run_fresh.argtypes = L.simc_arm_run.argtypes
     L.simc_arm_run_timed.argtypes = [_vp, C.c_int, C.POINTER(Settings), C.POINTER(EventsIn),
                                      C.POINTER(EventsOut), C.c_int64, C.POINTER(Rng), _vp,
                                      C.POINTER(_vp)]
     L.simc_recon_run.argtypes = [_vp, C.c_int, C.c_int64] + [_vp] * 9 + [_vp]
     L.simc_batch_create.argtypes = [_vp, C.POINTER(Setting), C.c_int, C.POINTER(_vp)]
     L.simc_batch_run.argtypes = [_vp, C.POINTER(EventsIn), C.POINTER(EventsOut), _vp]
+    L.simc_batch_run_fresh.argtypes = L.simc_batch_run.argtypes
     L.simc_batch_counters.argtypes = [_vp, C.c_int, C.POINTER(C.c_int64), C.c_int]
     L.simc_batch_set_chunk.argtypes = [_vp, C.c_int64]
     L.simc_batch_tune.argtypes = [_vp, C.POINTER(EventsIn), C.POINTER(EventsOut), _vp,
@@ -279,6 +282,7 @@ def library(path: str = LIB_PATH):
     L.simc_batch_passes.argtypes = [_vp, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
     L.simc_arm_run_host.argtypes = [_vp, C.c_int, C.POINTER(Settings), C.POINTER(EventsIn),
                                     C.POINTER(EventsOut), C.c_int64, C.POINTER(Rng)]
+    L.simc_arm_run_host_fresh.argtypes = L.simc_arm_run_host.argtypes
     L.simc_recon_run_host.argtypes = [_vp, C.c_int, C.c_int64] + [_vp] * 9
     L.simc_counters_get.argtypes = [_vp, C.c_int, C.POINTER(C.c_int64), C.c_int]
     L.simc_counters_reset.argtypes = [_vp, C.c_int]
@@ -326,6 +330,15 @@ def _dev_tensor(t, n, name, dtype, at_least=False):
     if not t.is_contiguous() or (t.numel() < n if at_least else t.numel() != n):
         raise ValueError(f"{name}: expected {'at least ' if at_least else ''}{n} contiguous elements")
     return t
+
+
+_NEW_DTYPES = {"ok": np.uint8, "stop": np.uint8, "used": np.int32}
+
+
+def _new_outputs(n, dev):
+    """Uninitialised device columns for the entries that write them whole."""
+    kinds = {"ok": torch.uint8, "stop": torch.uint8, "used": torch.int32}
+    return {k: torch.empty(n, dtype=kinds.get(k, torch.float64), device=dev) for k in OUT_FIELDS}
 
 
 def _check_outputs(out, n, required, at_least=False):
@@ -398,7 +411,13 @@ class Spectrometers:
         for k in ("z", "fry"):
             ev[k] = _dev_f64(events[k], n, k) if events.get(k) is not None else None
         dev = ev["dpp"].device
-        if out is None:
+        # New outputs are written whole by the kernels: neither cleared nor
+        # copied first (14 launches a call).  The sieve's forced angles and the
+        # timed entry keep the INOUT form.
+        fresh = out is None and not sieve and stage_events is None
+        if fresh:
+            out = _new_outputs(n, dev)
+        elif out is None:
             out = {k: ev[k].clone() for k in ("dpp", "y", "dxdz", "dydz")}
             for k in ("x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "resmult", "m2"):
                 out[k] = torch.zeros(n, dtype=torch.float64, device=dev)
@@ -420,8 +439,8 @@ class Spectrometers:
             R = Rng(RNG_PHILOX, 0, int(seed), int(event0), None, 0)
         st = stream if stream is not None else torch.cuda.current_stream(dev).cuda_stream
         if stage_events is None:
-            _check(library().simc_arm_run(self._h, arm, C.byref(S), C.byref(ein), C.byref(eout), n,
-                                          C.byref(R), C.c_void_p(st)))
+            entry = library().simc_arm_run_fresh if fresh else library().simc_arm_run
+            _check(entry(self._h, arm, C.byref(S), C.byref(ein), C.byref(eout), n, C.byref(R), C.c_void_p(st)))
         else:
             if len(stage_events) != 5 or any(e.cuda_event == 0 for e in stage_events):
                 raise ValueError("stage_events: five events, each recorded once beforehand")
@@ -440,7 +459,10 @@ class Spectrometers:
         n = len(events["dpp"])
         ev = {k: np.ascontiguousarray(events[k], dtype=np.float64) for k in
               ("dpp", "x", "y", "z", "dxdz", "dydz", "fry") if events.get(k) is not None}
-        if out is None:
+        fresh = out is None and not sieve
+        if fresh:  # written whole by the library
+            out = {k: np.empty(n, _NEW_DTYPES.get(k, np.float64)) for k in OUT_FIELDS}
+        elif out is None:
             out = {k: ev[k].copy() for k in ("dpp", "y", "dxdz", "dydz")}
             for k in ("x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "resmult", "m2"):
                 out[k] = np.zeros(n)
@@ -461,8 +483,8 @@ class Spectrometers:
             R = Rng(RNG_TAPE, 0, 0, event0, hp(tape), int(stride))
         else:
             R = Rng(RNG_PHILOX, 0, int(seed), int(event0), None, 0)
-        _check(library().simc_arm_run_host(self._h, arm, C.byref(S), C.byref(ein), C.byref(eout), n,
-                                           C.byref(R)))
+        entry = library().simc_arm_run_host_fresh if fresh else library().simc_arm_run_host
+        _check(entry(self._h, arm, C.byref(S), C.byref(ein), C.byref(eout), n, C.byref(R)))
         return out
 
     def recon_coefficients(self, arm):
@@ -971,11 +993,26 @@ class Batch:
         out["stop"] = torch.zeros(n, dtype=torch.uint8, device=dev)
         return out
 
+    def _covers(self, n):
+        """The settings' ranges are [0, n) without gaps or overlaps, and none uses the sieve."""
+        at = 0
+        for off, count in sorted((int(d["offset"]), int(d["count"])) for d in self.settings if int(d["count"])):
+            if off != at:
+                return False
+            at += count
+        return at == n and not any(d.get("sieve", 0) for d in self.settings)
+
     def run(self, events, out=None, stream=None):
-        out = self.new_outputs(events) if out is None else out
+        fresh = out is None and self._covers(events["dpp"].numel())
+        if fresh:  # written whole by the kernels
+            new = _new_outputs(events["dpp"].numel(), events["dpp"].device)
+            out = {k: new[k] for k in ("dpp", "y", "dxdz", "dydz", "x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "ok", "stop")}
+        elif out is None:
+            out = self.new_outputs(events)
         ein, eout = self._structs(events, out)
         st = stream if stream is not None else torch.cuda.current_stream(events["dpp"].device).cuda_stream
-        _check(library().simc_batch_run(self._h, C.byref(ein), C.byref(eout), C.c_void_p(st)))
+        entry = library().simc_batch_run_fresh if fresh else library().simc_batch_run
+        _check(entry(self._h, C.byref(ein), C.byref(eout), C.c_void_p(st)))
         return out
 
     def counters(self, i):

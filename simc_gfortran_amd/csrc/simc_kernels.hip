@@ -103,7 +103,10 @@ struct KArgs {
     uint32_t stride_bytes;
     unsigned long long* hist;   // per-setting histograms of kHistSlots bins
 };
-enum : int32_t { KF_MS = 1, KF_WCS = 2, KF_DECAY = 4, KF_COLL = 8, KF_FIT_F32 = 16, KF_SIEVE = 32, KF_SIEVE2 = 64 };
+enum : int32_t { KF_MS = 1, KF_WCS = 2, KF_DECAY = 4, KF_COLL = 8, KF_FIT_F32 = 16, KF_SIEVE = 32, KF_SIEVE2 = 64,
+              // the outputs are new: the INOUT columns (pathlen, resmult, x_fp..dy_fp) start from 0
+              // instead of what they hold, and every column is written for every event
+              KF_FRESH = 128 };
 
 typedef const double __attribute__((address_space(4)))* cdptr;
 typedef const Op __attribute__((address_space(4)))* coptr;
@@ -532,7 +535,7 @@ struct Hut {
     double& resmult;
     int scincount;
     ThetaCache ms;
-    double fp[4];  // fitted x_fp, x'_fp, y_fp, y'_fp
+    double (&fp)[4];  // fitted x_fp, x'_fp, y_fp, y'_fp
 
     // parameter j of program step k, for the parameters that depend on the maps
     __device__ __forceinline__ double runtime_p(int k, int j) const { return ((coptr)a.ops)[k].p[j]; }
@@ -684,18 +687,18 @@ __device__ __forceinline__ int hut_steps(H& h)
 // it waits for the step records' scalar loads).
 template <int ARM, class R, bool RARE, class S>
 __device__ __forceinline__ int hut_path(R& g, S& hs, Track& t, const KArgs& a, const Flags& F, uint32_t off,
-                                        double* lds_hits, double& resmult, int pc)
+                                        double* lds_hits, double& resmult, int pc, double (&fp)[4])
 {
     ThetaCache ms;
     ms.set(t);
     if constexpr (!RARE) {
         const bool plain = fabs(t.dxdzs) < 1.e6 && fabs(t.dydzs) < 1.e6 && ms.a < 1.e6 && fabs(ms.lb) < 1.e6;
         if (__all(plain)) {
-            Hut<ARM, R, RARE, S, false> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ms, {0.0, 0.0, 0.0, 0.0}};
+            Hut<ARM, R, RARE, S, false> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ms, fp};
             return hut_steps<ARM>(h);
         }
     }
-    Hut<ARM, R, RARE, S, true> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ms, {0.0, 0.0, 0.0, 0.0}};
+    Hut<ARM, R, RARE, S, true> h{g, hs, t, a, F, off, lds_hits, resmult, 0, ms, fp};
     return h.loop(pc);
 }
 
@@ -703,7 +706,7 @@ __device__ __forceinline__ int hut_path(R& g, S& hs, Track& t, const KArgs& a, c
 // the uniforms taken from the hut's own stream.
 template <int ARM, class R, bool RARE>
 __device__ __forceinline__ int run_hut(R& g, Track& t, const KArgs& a, const Flags& FA, uint32_t off,
-                                       double* lds_hits, double& resmult, uint32_t& drawn, int pc)
+                                       double* lds_hits, double& resmult, uint32_t& drawn, int pc, double (&fp)[4])
 {
     Flags F = FA;
     if (!RARE) {  // in-flight decay only in the RARE variant (as in the magnets)
@@ -714,12 +717,12 @@ __device__ __forceinline__ int run_hut(R& g, Track& t, const KArgs& a, const Fla
     if constexpr (HutStreamOf<R>::kOwn) {
         S hs;
         hs.init_from(g);
-        const int st = hut_path<ARM, R, RARE, S>(g, hs, t, a, F, off, lds_hits, resmult, pc);
+        const int st = hut_path<ARM, R, RARE, S>(g, hs, t, a, F, off, lds_hits, resmult, pc, fp);
         drawn = hs.used();
         return st;
     } else {
         drawn = 0;
-        return hut_path<ARM, R, RARE, R>(g, g, t, a, F, off, lds_hits, resmult, pc);
+        return hut_path<ARM, R, RARE, R>(g, g, t, a, F, off, lds_hits, resmult, pc, fp);
     }
 }
 
@@ -816,10 +819,11 @@ __device__ __forceinline__ void reconstruct_event(const KArgs& a, uint32_t off)
 
 // Outputs of a finished event (byte offset off in the event arrays); an
 // accepted event is reconstructed here unless RECON_LATER (the hut stage
-// hands accepted events to recon_list_kernel).
+// hands accepted events to recon_list_kernel).  fp: the fitted track (0 before
+// the fit); accepted events' is stored at the fit.
 template <int ARM, bool RECON_LATER = false>
 __device__ __forceinline__ void finish_event(const KArgs& a, uint32_t off, int st, uint32_t used, const Track& t,
-                                             double resmult)
+                                             double resmult, const double (&fp)[4])
 {
     const uint32_t n = a.n_arr;
     if (st == ST_OK) {
@@ -832,6 +836,12 @@ __device__ __forceinline__ void finish_event(const KArgs& a, uint32_t off, int s
         if (!(a.flags & (KF_SIEVE | KF_SIEVE2))) {
             st64(a.o_dxdz, n, off, ld64(a.dxdz, n, off));
             st64(a.o_dydz, n, off, ld64(a.dydz, n, off));
+        }
+        if (a.flags & KF_FRESH) {  // the fitted track, or 0 where the fit was not reached
+            st64(a.x_fp, n, off, fp[0]);
+            st64(a.dx_fp, n, off, fp[1]);
+            st64(a.y_fp, n, off, fp[2]);
+            st64(a.dy_fp, n, off, fp[3]);
         }
     }
     st64(a.pathlen, n, off, t.pathlen);
@@ -946,7 +956,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2
             t.dflag = (int)(bits & 1u);
             // resmult is drawn in the hut only: until then it is the
             // caller's INOUT value, still in place at the event's index
-            resmult = a.resmult ? ld64(a.resmult, a.n_arr, e.off) : 0.0;
+            resmult = a.resmult && !(a.flags & KF_FRESH) ? ld64(a.resmult, a.n_arr, e.off) : 0.0;
         } else {
             li = i;
             s = find_setting(a, a.pass_base + li);
@@ -964,14 +974,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2
             t.dpps = ld64(a.dpp, n, off);
             t.p = S.p_spec * (1.0 + t.dpps / 100.0);
             t.m2 = S.m2;
-            t.pathlen = ld64(a.pathlen, n, off);
+            t.pathlen = a.flags & KF_FRESH ? 0.0 : ld64(a.pathlen, n, off);
             t.decdist = 0.0;
             t.dflag = 0;
-            resmult = a.resmult ? ld64(a.resmult, n, off) : 0.0;
+            resmult = a.resmult && !(a.flags & KF_FRESH) ? ld64(a.resmult, n, off) : 0.0;
         }
         int st;
         uint32_t hut_drawn = 0;
-        if constexpr (STAGE == STAGE_HUT) st = run_hut<ARM, R, RARE>(g, t, a, F, e.off, lds_hits, resmult, hut_drawn, pc_begin);
+        double fp[4] = {0.0, 0.0, 0.0, 0.0};
+        if constexpr (STAGE == STAGE_HUT) st = run_hut<ARM, R, RARE>(g, t, a, F, e.off, lds_hits, resmult, hut_drawn, pc_begin, fp);
         else if constexpr (!FROM_Q && !kTranspBeforeCollimator<ARM>)
             st = run_program<ARM, R, RARE, false, false>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
         else if (a.gen) st = run_program<ARM, R, RARE, true, true>(g, t, a, F, e.off, coll_cnt, pc_begin, pc_end);
@@ -980,13 +991,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2
         if (g.overflow) st = ST_TAPE;
         if (STAGE == STAGE_HUT) {
             // TO_Q: accepted events go to the reconstruction list
-            finish_event<ARM, TO_Q>(a, e.off, st, used, t, resmult);
+            finish_event<ARM, TO_Q>(a, e.off, st, used, t, resmult, fp);
             count_stop(a, hist, s_block, s, st);
             survivor = TO_Q && st == ST_OK;
         } else if (TO_Q && st == ST_OK) {
             survivor = true;
         } else {
-            finish_event<ARM>(a, e.off, st, used, t, resmult);
+            finish_event<ARM>(a, e.off, st, used, t, resmult, fp);
             count_stop(a, hist, s_block, s, st);
         }
         if (coll_cnt[0] | coll_cnt[1] | coll_cnt[2]) {
@@ -2664,9 +2675,11 @@ int launch_stages(simc_ctx* ctx, int arm, bool rare, bool tape, const KArgs& a, 
 }
 
 // fixed: the queue pair to use (room for n events), or nullptr for the
-// context's queues of the arm (grown here as needed).
+// context's queues of the arm (grown here as needed).  fresh: the outputs
+// hold nothing (KF_FRESH).
 int arm_run(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in, simc_events_out* out,
-            int64_t n, const simc_rng* rng, void* stream, void* const* stage_events, const Queue* fixed = nullptr)
+            int64_t n, const simc_rng* rng, void* stream, void* const* stage_events, const Queue* fixed = nullptr,
+            bool fresh = false)
 {
     if (!ctx || !s || !in || !out || !rng) return fail(SIMC_E_ARG, "simc_arm_run: NULL argument");
     const int ai = arm_index(arm);
@@ -2684,7 +2697,7 @@ int arm_run(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in
     a.set0 = make_setdev(arm, s, rng->seed, rng->event0, 0, 0, 0);
     a.set = nullptr;
     a.n_set = 1;
-    a.flags = a.set0.flags;
+    a.flags = a.set0.flags | (fresh ? KF_FRESH : 0);
     a.seed = rng->seed;
     a.tab = ctx->d_tab[ai];
     a.coef = ctx->d_coef[ai];
@@ -2749,6 +2762,13 @@ int simc_arm_run(simc_ctx* ctx, int arm, const simc_settings* s, const simc_even
     return arm_run(ctx, arm, s, in, out, n, rng, stream, nullptr);
 }
 
+int simc_arm_run_fresh(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in,
+                       simc_events_out* out, int64_t n, const simc_rng* rng, void* stream)
+{
+    if (s && s->sieve) return fail(SIMC_E_ARG, "simc_arm_run_fresh: not with the mock sieve (its angles are INOUT)");
+    return arm_run(ctx, arm, s, in, out, n, rng, stream, nullptr, nullptr, true);
+}
+
 int simc_arm_run_noalloc(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in,
                          simc_events_out* out, int64_t n, const simc_rng* rng, void* stream)
 {
@@ -2773,8 +2793,8 @@ int simc_arm_run_timed(simc_ctx* ctx, int arm, const simc_settings* s, const sim
     return arm_run(ctx, arm, s, in, out, n, rng, stream, stage_events);
 }
 
-int simc_arm_run_host(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in,
-                      simc_events_out* out, int64_t n, const simc_rng* rng)
+static int arm_run_host(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in,
+                        simc_events_out* out, int64_t n, const simc_rng* rng, bool fresh)
 {
     if (!ctx || !s || !in || !out || !rng) return fail(SIMC_E_ARG, "simc_arm_run_host: NULL argument");
     if (n < 0) return fail(SIMC_E_ARG, "negative event count");
@@ -2799,8 +2819,8 @@ int simc_arm_run_host(simc_ctx* ctx, int arm, const simc_settings* s, const simc
     const size_t n_in = cols.size();
     double* hio[6] = {out->x_fp, out->dx_fp, out->y_fp, out->dy_fp, out->pathlen, out->resmult};
     for (double* p : hio)
-        if (p) cols.push_back({p, p, 8});
-    const size_t n_io = cols.size() - n_in;
+        if (p) cols.push_back({fresh ? nullptr : p, p, 8});
+    const size_t n_io = fresh ? 0 : cols.size() - n_in;
     double* hw[5] = {out->dpp, out->y, out->dxdz, out->dydz, out->m2};
     for (double* p : hw)
         if (p) cols.push_back({nullptr, p, 8});
@@ -2957,7 +2977,7 @@ int simc_arm_run_host(simc_ctx* ctx, int arm, const simc_settings* s, const simc
         if (tape) drng.tape = (const double*)(d + tape_off);
         else drng.event0 = rng->event0 + (uint64_t)c0;
         Queue fq[2] = {q1[j], q2[j]};  // the slot's own queues: two chunks are in flight at once
-        rc = arm_run(ctx, arm, s, &ein, &eout, m, &drng, (void*)st, nullptr, fq);
+        rc = arm_run(ctx, arm, s, &ein, &eout, m, &drng, (void*)st, nullptr, fq, fresh);
         if (rc) break;
         HIPCHK(hipMemcpyAsync((char*)hp.pinned[j] + out_beg, d + out_beg, out_end - out_beg, hipMemcpyDeviceToHost,
                               st));
@@ -2975,6 +2995,19 @@ int simc_arm_run_host(simc_ctx* ctx, int arm, const simc_settings* s, const simc
         return rc;
     }
     return SIMC_OK;
+}
+
+int simc_arm_run_host(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in,
+                      simc_events_out* out, int64_t n, const simc_rng* rng)
+{
+    return arm_run_host(ctx, arm, s, in, out, n, rng, false);
+}
+
+int simc_arm_run_host_fresh(simc_ctx* ctx, int arm, const simc_settings* s, const simc_events_in* in,
+                            simc_events_out* out, int64_t n, const simc_rng* rng)
+{
+    if (s && s->sieve) return fail(SIMC_E_ARG, "simc_arm_run_host_fresh: not with the mock sieve (its angles are INOUT)");
+    return arm_run_host(ctx, arm, s, in, out, n, rng, true);
 }
 
 int simc_recon_run_host(simc_ctx* ctx, int arm, int64_t n, const double* x_fp, const double* dx_fp,
@@ -4203,7 +4236,7 @@ int simc_batch_set_chunk(simc_batch* b, int64_t chunk)
     return SIMC_OK;
 }
 
-int simc_batch_run(simc_batch* b, const simc_events_in* in, simc_events_out* out, void* stream)
+static int batch_run(simc_batch* b, const simc_events_in* in, simc_events_out* out, void* stream, bool fresh)
 {
     if (!b || !in || !out) return fail(SIMC_E_ARG, "simc_batch_run: NULL argument");
     if (!outputs_complete(in, out)) return fail(SIMC_E_ARG, "missing event input or output array");
@@ -4223,7 +4256,7 @@ int simc_batch_run(simc_batch* b, const simc_events_in* in, simc_events_out* out
         std::memset(&a, 0, sizeof a);
         a.set = (const SetDev*)b->d_set + pass.first;
         a.n_set = pass.n;
-        a.flags = pass.flags;
+        a.flags = pass.flags | (fresh ? KF_FRESH : 0);
         a.seed = pass.seed;
         a.ix_base = 0;
         a.n_arr = b->n_arr;
@@ -4245,6 +4278,20 @@ int simc_batch_run(simc_batch* b, const simc_events_in* in, simc_events_out* out
         }
     }
     return SIMC_OK;
+}
+
+int simc_batch_run(simc_batch* b, const simc_events_in* in, simc_events_out* out, void* stream)
+{
+    return batch_run(b, in, out, stream, false);
+}
+
+int simc_batch_run_fresh(simc_batch* b, const simc_events_in* in, simc_events_out* out, void* stream)
+{
+    if (b)
+        for (const auto& pass : b->passes)
+            if (pass.flags & (KF_SIEVE | KF_SIEVE2))
+                return fail(SIMC_E_ARG, "simc_batch_run_fresh: not with the mock sieve (its angles are INOUT)");
+    return batch_run(b, in, out, stream, true);
 }
 
 int simc_batch_passes(simc_batch* b, int32_t* n_passes, int32_t* n_lane_key)
