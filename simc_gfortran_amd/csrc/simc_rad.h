@@ -72,6 +72,13 @@ __device__ __noinline__ double rad_inter(double alpha, double ar1, double ar2, d
     return r * amult / kPi;
 }
 
+// gamma, out of line: the generator calls it 24 times, and with an inlined
+// copy at each the kernel was 739 KB of code, eleven times the instruction
+// cache (1e6 events: 1.46 -> 1.32 ms, fewer values in scratch, same bits).
+// Powers and logarithms out of line as well gave nothing more: the registers
+// saved around the calls cost what the code saves.
+__device__ __noinline__ double rad_tgamma(double x) { return tgamma(x); }
+
 // inter_prime, brem.f:581-598
 __device__ __forceinline__ double rad_inter_prime(double alpha, double ar1, double ar2, double de)
 {
@@ -283,25 +290,25 @@ __device__ __forceinline__ void rad_basicrad_init_ev(RadState& S, double e1, dou
     ci[1] = lam[0] / pow(e1 * e2, lam[0] / 2.);
     ci[2] = lam[1] / pow(e1 * e2, lam[1] / 2.);
     ci[3] = lam[2] / pow(kMp * e3, lam[2] / 2.);
-    for (int i = 1; i <= 3; ++i) ci[i] = ci[i] * exp(-kEuler * lam[i - 1]) / tgamma(one + lam[i - 1]);
+    for (int i = 1; i <= 3; ++i) ci[i] = ci[i] * exp(-kEuler * lam[i - 1]) / rad_tgamma(one + lam[i - 1]);
     S.g_int = lam[0] + lam[1] + lam[2];
     ci[0] = ci[1] * ci[2] * S.g_int / lam[0] / lam[1];
     if (lam[2] > 0) ci[0] = ci[0] * ci[3] / lam[2];
-    ci[0] = ci[0] * tgamma(one + lam[0]) * tgamma(one + lam[1]) * tgamma(one + lam[2]) / tgamma(one + S.g_int);
-    ce[1] = bt[0] / pow(e1, bt[0]) / tgamma(one + bt[0]);
-    ce[2] = bt[1] / pow(e2, bt[1]) / tgamma(one + bt[1]);
+    ci[0] = ci[0] * rad_tgamma(one + lam[0]) * rad_tgamma(one + lam[1]) * rad_tgamma(one + lam[2]) / rad_tgamma(one + S.g_int);
+    ce[1] = bt[0] / pow(e1, bt[0]) / rad_tgamma(one + bt[0]);
+    ce[2] = bt[1] / pow(e2, bt[1]) / rad_tgamma(one + bt[1]);
     ce[3] = 0.0;
     S.g_ext = bt[0] + bt[1];
     ce[0] = ce[1] * ce[2] * S.g_ext / bt[0] / bt[1];
-    ce[0] = ce[0] * tgamma(one + bt[0]) * tgamma(one + bt[1]) / tgamma(one + S.g_ext);
+    ce[0] = ce[0] * rad_tgamma(one + bt[0]) * rad_tgamma(one + bt[1]) / rad_tgamma(one + S.g_ext);
     for (int i = 1; i <= 2; ++i)
-        c[i] = ci[i] * ce[i] * g[i] / lam[i - 1] / bt[i - 1] * tgamma(one + lam[i - 1]) * tgamma(one + bt[i - 1]) /
-               tgamma(one + g[i]);
+        c[i] = ci[i] * ce[i] * g[i] / lam[i - 1] / bt[i - 1] * rad_tgamma(one + lam[i - 1]) * rad_tgamma(one + bt[i - 1]) /
+               rad_tgamma(one + g[i]);
     c[3] = ci[3];
     c[0] = c[1] * c[2] * g[0] / g[1] / g[2];
     if (g[3] > 0) c[0] = c[0] * c[3] / g[3];
-    c[0] = c[0] * tgamma(one + g[1]) * tgamma(one + g[2]) * tgamma(one + g[3]) / tgamma(one + g[0]);
-    c[4] = g[4] / pow(e1 * e2, g[4]) / tgamma(one + g[4]);
+    c[0] = c[0] * rad_tgamma(one + g[1]) * rad_tgamma(one + g[2]) * rad_tgamma(one + g[3]) / rad_tgamma(one + g[0]);
+    c[4] = g[4] / pow(e1 * e2, g[4]) / rad_tgamma(one + g[4]);
     if (g[3] > 0) c[4] = c[4] / pow(e3, g[4]);
 }
 
@@ -389,7 +396,7 @@ __device__ __forceinline__ double rad_extrad_phi(const RadDev& R, const RadState
         const double x = Egamma / (itail == 1 ? E1 : E2);
         const double t = S.bt[itail - 1] / R.etatzai;
         phi = phi * (1. - x + (x * x) / R.etatzai) * exp(t * ((R.etatzai - 0.5) - R.etatzai * x + (x * x) / 2.)) *
-              tgamma(1. + S.bt[itail - 1]);
+              rad_tgamma(1. + S.bt[itail - 1]);
     }
     return phi;
 }
@@ -420,8 +427,8 @@ __device__ __forceinline__ double rad_peaked_weight(const RadDev& R, const RadSt
         w = S.c_ext[0] / S.g_ext * (exp(-dsoft_intmax) * pow(emax, S.g_ext));
     const double* g = S.g;
     const double* bt = S.bt;
-    w = w * exp(-eul * g[4]) / tgamma(1. + g[4]) * tgamma(1. + g[4] - bt[0] - bt[1]) * tgamma(1. + bt[0]) *
-        tgamma(1. + bt[1]) / tgamma(1. + g[4]);
+    w = w * exp(-eul * g[4]) / rad_tgamma(1. + g[4]) * rad_tgamma(1. + g[4] - bt[0] - bt[1]) * rad_tgamma(1. + bt[0]) *
+        rad_tgamma(1. + bt[1]) / rad_tgamma(1. + g[4]);
     if (w < 0) w = 0;
     return w;
 }
