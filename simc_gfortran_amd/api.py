@@ -967,6 +967,14 @@ class Batch:
         self.ctx = ctx
         self.settings = list(settings)
         self.n_arr = max(int(d["offset"]) + int(d["count"]) for d in settings)
+        # length of the arrays that the settings' ranges cover without gaps or
+        # overlaps, or None (also with the sieve, whose angles are INOUT)
+        at = 0
+        for off, count in sorted((int(d["offset"]), int(d["count"])) for d in settings if int(d["count"])):
+            at = at + count if off == at else -1
+            if at < 0:
+                break
+        self._whole = None if at < 0 or any(d.get("sieve", 0) for d in settings) else at
         h = _vp()
         _check(library().simc_batch_create(ctx._h, arr, len(settings), C.byref(h)))
         self._h = h
@@ -993,17 +1001,8 @@ class Batch:
         out["stop"] = torch.zeros(n, dtype=torch.uint8, device=dev)
         return out
 
-    def _covers(self, n):
-        """The settings' ranges are [0, n) without gaps or overlaps, and none uses the sieve."""
-        at = 0
-        for off, count in sorted((int(d["offset"]), int(d["count"])) for d in self.settings if int(d["count"])):
-            if off != at:
-                return False
-            at += count
-        return at == n and not any(d.get("sieve", 0) for d in self.settings)
-
     def run(self, events, out=None, stream=None):
-        fresh = out is None and self._covers(events["dpp"].numel())
+        fresh = out is None and self._whole == events["dpp"].numel()
         if fresh:  # written whole by the kernels
             new = _new_outputs(events["dpp"].numel(), events["dpp"].device)
             out = {k: new[k] for k in ("dpp", "y", "dxdz", "dydz", "x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "ok", "stop")}

@@ -308,6 +308,19 @@ module simc_gpu
       type(simc_rng), intent(in) :: rng
     end function
 
+    ! into outputs that hold nothing yet: INOUT columns start from 0, every column is written
+    integer(c_int) function simc_arm_run_fresh(ctx, arm, s, evin, evout, n, rng, stream) &
+        bind(C, name="simc_arm_run_fresh")
+      import :: c_int, c_int64_t, c_ptr, simc_settings, simc_events_in, simc_events_out, simc_rng
+      type(c_ptr), value :: ctx, stream
+      integer(c_int), value :: arm
+      type(simc_settings), intent(in) :: s
+      type(simc_events_in), intent(in) :: evin
+      type(simc_events_out), intent(in) :: evout
+      integer(c_int64_t), value :: n
+      type(simc_rng), intent(in) :: rng
+    end function
+
     ! allocation-free variant: at most SIMC_NOALLOC_MAX_EVENTS (524288) events per call
     integer(c_int) function simc_arm_run_noalloc(ctx, arm, s, evin, evout, n, rng, stream) &
         bind(C, name="simc_arm_run_noalloc")
@@ -372,6 +385,19 @@ module simc_gpu
     end function
 
     integer(c_int) function simc_arm_run_host(ctx, arm, s, evin, evout, n, rng) bind(C, name="simc_arm_run_host")
+      import :: c_int, c_int64_t, c_ptr, simc_settings, simc_events_in, simc_events_out, simc_rng
+      type(c_ptr), value :: ctx
+      integer(c_int), value :: arm
+      type(simc_settings), intent(in) :: s
+      type(simc_events_in), intent(in) :: evin
+      type(simc_events_out), intent(in) :: evout
+      integer(c_int64_t), value :: n
+      type(simc_rng), intent(in) :: rng
+    end function
+
+    ! the same on host arrays
+    integer(c_int) function simc_arm_run_host_fresh(ctx, arm, s, evin, evout, n, rng) &
+        bind(C, name="simc_arm_run_host_fresh")
       import :: c_int, c_int64_t, c_ptr, simc_settings, simc_events_in, simc_events_out, simc_rng
       type(c_ptr), value :: ctx
       integer(c_int), value :: arm
@@ -479,6 +505,15 @@ module simc_gpu
     end function
 
     integer(c_int) function simc_batch_run(b, evin, evout, stream) bind(C, name="simc_batch_run")
+      import :: c_int, c_ptr, simc_events_in, simc_events_out
+      type(c_ptr), value :: b, stream
+      type(simc_events_in), intent(in) :: evin
+      type(simc_events_out), intent(in) :: evout
+    end function
+
+    ! the same for a batch
+    integer(c_int) function simc_batch_run_fresh(b, evin, evout, stream) &
+        bind(C, name="simc_batch_run_fresh")
       import :: c_int, c_ptr, simc_events_in, simc_events_out
       type(c_ptr), value :: b, stream
       type(simc_events_in), intent(in) :: evin
