@@ -335,10 +335,9 @@ def _dev_tensor(t, n, name, dtype, at_least=False):
 _NEW_DTYPES = {"ok": np.uint8, "stop": np.uint8, "used": np.int32}
 
 
-def _new_outputs(n, dev):
+def _new_outputs(n, dev, columns=OUT_FIELDS):
     """Uninitialised device columns for the entries that write them whole."""
-    kinds = {"ok": torch.uint8, "stop": torch.uint8, "used": torch.int32}
-    return {k: torch.empty(n, dtype=kinds.get(k, torch.float64), device=dev) for k in OUT_FIELDS}
+    return {k: torch.empty(n, dtype=OUT_DTYPES[k], device=dev) for k in columns}
 
 
 def _check_outputs(out, n, required, at_least=False):
@@ -1004,8 +1003,7 @@ class Batch:
     def run(self, events, out=None, stream=None):
         fresh = out is None and self._whole == events["dpp"].numel()
         if fresh:  # written whole by the kernels
-            new = _new_outputs(events["dpp"].numel(), events["dpp"].device)
-            out = {k: new[k] for k in ("dpp", "y", "dxdz", "dydz", "x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "ok", "stop")}
+            out = _new_outputs(events["dpp"].numel(), events["dpp"].device, RUN_REQUIRED)
         elif out is None:
             out = self.new_outputs(events)
         ein, eout = self._structs(events, out)

@@ -68,3 +68,24 @@ def test_batch_with_a_gap_keeps_the_cleared_form(ctx):
         np.testing.assert_array_equal(gap, ev[k][1000:1500].cpu().numpy() if k in ev else np.zeros_like(gap), err_msg=k)
         for sl in (slice(0, 1000), slice(1500, 3000)):
             np.testing.assert_array_equal(out[k][sl].cpu().numpy(), full[k][sl].cpu().numpy(), err_msg=k)
+
+
+def test_batch_allocates_only_the_columns_it_returns(ctx):
+    """A batch's outputs are what the call takes: 74 bytes an event, and
+    nothing else for its duration."""
+    from simc_gfortran_amd import api
+    wl, n = W.HMS_C0, 2_000_000
+    ev = W.generate_device(wl, n, seed=4, device=torch.device("cuda"))
+    b = api.Batch(ctx, [dict(arm=wl.arm, p_spec=wl.p_spec, m2=wl.m2, seed=1, offset=0, count=n)])
+    b.run(ev)  # the library's own queues
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = b.run(ev)
+    torch.cuda.synchronize()
+    peak = torch.cuda.max_memory_allocated() - before
+    returned = sum(v.numel() * v.element_size() for v in out.values())
+    assert returned == 74 * n
+    # a block's unsplit remainder is less than 1 MiB: eleven are less than one more column, 16 MB
+    assert peak < returned + 8 * n, (peak, returned)
