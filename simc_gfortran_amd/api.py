@@ -92,6 +92,8 @@ class EventsIn(C.Structure):
 
 OUT_FIELDS = ("dpp", "y", "dxdz", "dydz", "x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen",
               "resmult", "m2", "ok", "stop", "used")
+# the outputs that start as the inputs of the same name
+INOUT = ("dpp", "y", "dxdz", "dydz")
 # the outputs a run always writes (resmult, m2 and used are optional)
 RUN_REQUIRED = ("dpp", "y", "dxdz", "dydz", "x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "ok", "stop")
 
@@ -458,6 +460,9 @@ class Spectrometers:
         n = len(events["dpp"])
         ev = {k: np.ascontiguousarray(events[k], dtype=np.float64) for k in
               ("dpp", "x", "y", "z", "dxdz", "dydz", "fry") if events.get(k) is not None}
+        for k, v in ev.items():  # the library reads n elements of each
+            if len(v) < n or (k in INOUT and len(v) != n):
+                raise TypeError(f"events[{k!r}]: expected {n} elements")
         fresh = out is None and not sieve
         if fresh:  # written whole by the library
             out = {k: np.empty(n, _NEW_DTYPES.get(k, np.float64)) for k in OUT_FIELDS}
