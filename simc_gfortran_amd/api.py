@@ -337,9 +337,12 @@ def _dev_tensor(t, n, name, dtype, at_least=False):
 _NEW_DTYPES = {"ok": np.uint8, "stop": np.uint8, "used": np.int32}
 
 
-def _new_outputs(n, dev, columns=OUT_FIELDS):
-    """Uninitialised device columns for the entries that write them whole."""
-    return {k: torch.empty(n, dtype=OUT_DTYPES[k], device=dev) for k in columns}
+def _new_outputs(events, columns=OUT_FIELDS):
+    """Uninitialised device columns for the entries that write them whole; the
+    INOUT ones have their inputs' shapes."""
+    n, dev = events["dpp"].numel(), events["dpp"].device
+    return {k: torch.empty_like(events[k]) if k in INOUT else torch.empty(n, dtype=OUT_DTYPES[k], device=dev)
+            for k in columns}
 
 
 def _check_outputs(out, n, required, at_least=False):
@@ -417,7 +420,7 @@ class Spectrometers:
         # timed entry keep the INOUT form.
         fresh = out is None and not sieve and stage_events is None
         if fresh:
-            out = _new_outputs(n, dev)
+            out = _new_outputs(ev)
         elif out is None:
             out = {k: ev[k].clone() for k in ("dpp", "y", "dxdz", "dydz")}
             for k in ("x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "resmult", "m2"):
@@ -465,7 +468,8 @@ class Spectrometers:
                 raise TypeError(f"events[{k!r}]: expected {n} elements")
         fresh = out is None and not sieve
         if fresh:  # written whole by the library
-            out = {k: np.empty(n, _NEW_DTYPES.get(k, np.float64)) for k in OUT_FIELDS}
+            out = {k: np.empty_like(ev[k]) if k in INOUT else np.empty(n, _NEW_DTYPES.get(k, np.float64))
+                   for k in OUT_FIELDS}
         elif out is None:
             out = {k: ev[k].copy() for k in ("dpp", "y", "dxdz", "dydz")}
             for k in ("x_fp", "dx_fp", "y_fp", "dy_fp", "pathlen", "resmult", "m2"):
@@ -1006,9 +1010,9 @@ class Batch:
         return out
 
     def run(self, events, out=None, stream=None):
-        fresh = out is None and self._whole == events["dpp"].numel()
+        fresh = out is None and all(self._whole == events[k].numel() for k in INOUT)
         if fresh:  # written whole by the kernels
-            out = _new_outputs(events["dpp"].numel(), events["dpp"].device, RUN_REQUIRED)
+            out = _new_outputs(events, RUN_REQUIRED)
         elif out is None:
             out = self.new_outputs(events)
         ein, eout = self._structs(events, out)

@@ -89,3 +89,26 @@ def test_batch_allocates_only_the_columns_it_returns(ctx):
     assert returned == 74 * n
     # a block's unsplit remainder is less than 1 MiB: eleven are less than one more column, 16 MB
     assert peak < returned + 8 * n, (peak, returned)
+
+
+def test_new_outputs_have_the_inputs_shape(ctx):
+    """dpp, y, dxdz and dydz come back in the shape of their inputs (as they do
+    when they start as copies of them), also a column longer than a batch."""
+    from simc_gfortran_amd import api
+    wl, n = W.SHMS_C1, 3000
+    inout = ("dpp", "y", "dxdz", "dydz")
+    flat = W.generate_device(wl, n, seed=4, device=torch.device("cuda"))
+    ev = {k: v.view(n // 3, 3) for k, v in flat.items()}
+    kw = dict(p_spec=wl.p_spec, m2=wl.m2, seed=1)
+    ref = ctx.run(wl.arm, flat, **kw)
+    b = api.Batch(ctx, [dict(arm=wl.arm, offset=0, count=n, **kw)])
+    host = {k: v.cpu().numpy().reshape(n, 1) for k, v in flat.items()}
+    long = dict(flat, y=torch.cat([flat["y"], flat["y"][:5]]))
+    for out in (ctx.run(wl.arm, ev, **kw), b.run(ev), ctx.run_host(wl.arm, host, **kw), b.run(long)):
+        out = {k: torch.as_tensor(v).cpu() for k, v in out.items()}
+        given = long if out["y"].numel() > n else host if out["y"].shape == (n, 1) else ev
+        for k in inout:
+            assert tuple(out[k].shape) == tuple(given[k].shape), k
+        for k in inout + ("x_fp", "pathlen", "ok"):
+            np.testing.assert_array_equal(out[k].reshape(-1)[:n].numpy(), ref[k].cpu().numpy(), err_msg=k)
+        np.testing.assert_array_equal(out["y"].reshape(-1)[n:].numpy(), flat["y"][:out["y"].numel() - n].cpu().numpy())
