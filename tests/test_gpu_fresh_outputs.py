@@ -112,3 +112,103 @@ def test_new_outputs_have_the_inputs_shape(ctx):
         for k in inout + ("x_fp", "pathlen", "ok"):
             np.testing.assert_array_equal(out[k].reshape(-1)[:n].numpy(), ref[k].cpu().numpy(), err_msg=k)
         np.testing.assert_array_equal(out["y"].reshape(-1)[n:].numpy(), flat["y"][:out["y"].numel() - n].cpu().numpy())
+
+
+JUNK = {"ok": 0xFF, "stop": 0xFF, "used": -7}
+ALL = [W.HMS_C0, W.SHMS_C1, W.SOS_1p5, W.HRSR_2, W.HRSL_3]
+E_ARG = -6  # SIMC_E_ARG
+
+
+def dirty(n):
+    """Host columns holding what no run writes."""
+    from simc_gfortran_amd import api
+    kinds = {"ok": np.uint8, "stop": np.uint8, "used": np.int32}
+    return {k: np.full(n, JUNK.get(k, np.nan), kinds.get(k, np.float64)) for k in api.OUT_FIELDS}
+
+
+def structs(api, ev, out, ptr):
+    return (api.EventsIn(*[ptr(ev.get(k)) for k in ("dpp", "x", "y", "z", "dxdz", "dydz", "fry")]),
+            api.EventsOut(*[ptr(out.get(k)) for k in api.OUT_FIELDS]))
+
+
+@pytest.mark.parametrize("rng", ["philox", "tape"])
+@pytest.mark.parametrize("wl", ALL, ids=lambda w: w.name)
+def test_every_column_of_dirty_outputs_is_written(ctx, wl, rng):
+    """The C entries on outputs full of junk give what the cleared form gives;
+    the tape is too short for the hut, so events end at it as well."""
+    import ctypes as C
+    from simc_gfortran_amd import api
+    L, n, dev, stride = api.library(), 5003, torch.device("cuda"), 120
+    ev = W.generate_device(wl, n, seed=6, device=dev)
+    host = {k: v.cpu().numpy() for k, v in ev.items()}
+    kw = dict(p_spec=wl.p_spec, m2=wl.m2, wire_sigma=wl.wire_sigma, fit="fp64")
+    S = api.Settings(wl.p_spec, wl.m2, 0.0, 1, 1, 0, 0, api.FIT_FP64, 0, wl.wire_sigma)
+    if rng == "tape":
+        tape = W.uniform_tape(n, stride, seed=3)
+        d_tape = torch.from_numpy(tape).to(dev)
+        old = ctx.run(wl.arm, ev, out=cleared(ev, n, dev), rng="tape", tape=d_tape, stride=stride, **kw)
+        R = api.Rng(api.RNG_TAPE, 0, 0, 0, d_tape.data_ptr(), stride)
+        RH = api.Rng(api.RNG_TAPE, 0, 0, 0, tape.ctypes.data, stride)
+    else:
+        old = ctx.run(wl.arm, ev, out=cleared(ev, n, dev), seed=9, **kw)
+        R = RH = api.Rng(api.RNG_PHILOX, 0, 9, 0, None, 0)
+    old = {k: v.cpu().numpy() for k, v in old.items()}
+    assert (old["stop"] == 250).any() == (rng == "tape")  # past the end of its tape
+
+    new = {k: torch.from_numpy(v).to(dev) for k, v in dirty(n).items()}
+    ein, eout = structs(api, ev, new, lambda t: None if t is None else t.data_ptr())
+    st = torch.cuda.current_stream().cuda_stream
+    assert L.simc_arm_run_fresh(ctx._h, wl.arm, C.byref(S), C.byref(ein), C.byref(eout), n, C.byref(R), C.c_void_p(st)) == 0
+    torch.cuda.synchronize()
+    got = dirty(n)
+    hin, hout = structs(api, host, got, lambda a: None if a is None else a.ctypes.data)
+    assert L.simc_arm_run_host_fresh(ctx._h, wl.arm, C.byref(S), C.byref(hin), C.byref(hout), n, C.byref(RH)) == 0
+    for k in old:
+        np.testing.assert_array_equal(new[k].cpu().numpy(), old[k], err_msg=k)
+        np.testing.assert_array_equal(got[k], old[k], err_msg="host " + k)
+
+
+def test_every_column_of_a_batch_is_written(ctx):
+    import ctypes as C
+    from simc_gfortran_amd import api
+    dev, n = torch.device("cuda"), 9001
+    ev = {k: torch.empty(n, dtype=torch.float64, device=dev) for k in ("dpp", "x", "y", "z", "dxdz", "dydz", "fry")}
+    at, table = 0, []
+    for i, wl in enumerate(ALL):
+        m = 2003 if i < 4 else n - at
+        W.generate_device(wl, m, seed=i, device=dev, out=ev, at=at)
+        table.append(dict(arm=wl.arm, p_spec=wl.p_spec, m2=wl.m2, wire_sigma=wl.wire_sigma, fit="fp64", seed=i,
+                          offset=at, count=m))
+        at += m
+    b = api.Batch(ctx, table)
+    old = b.run(ev, out=b.new_outputs(ev))
+    new = {k: torch.from_numpy(v).to(dev) for k, v in dirty(n).items() if k in old}
+    ein, eout = structs(api, ev, new, lambda t: None if t is None else t.data_ptr())
+    st = torch.cuda.current_stream().cuda_stream
+    assert api.library().simc_batch_run_fresh(b._h, C.byref(ein), C.byref(eout), C.c_void_p(st)) == 0
+    torch.cuda.synchronize()
+    for k in old:
+        np.testing.assert_array_equal(new[k].cpu().numpy(), old[k].cpu().numpy(), err_msg=k)
+
+
+def test_the_sieve_is_refused(ctx):
+    """Its forced angles are INOUT; the outputs stay as they are."""
+    import ctypes as C
+    from simc_gfortran_amd import api
+    L, wl, n, dev = api.library(), W.HMS_C0, 300, torch.device("cuda")
+    ev = W.generate_device(wl, n, seed=6, device=dev)
+    host = {k: v.cpu().numpy() for k, v in ev.items()}
+    S = api.Settings(wl.p_spec, wl.m2, 0.0, 1, 1, 0, 0, api.FIT_FP64, 1, wl.wire_sigma)
+    R = api.Rng(api.RNG_PHILOX, 0, 9, 0, None, 0)
+    new, got = {k: torch.from_numpy(v).to(dev) for k, v in dirty(n).items()}, dirty(n)
+    ein, eout = structs(api, ev, new, lambda t: None if t is None else t.data_ptr())
+    hin, hout = structs(api, host, got, lambda a: None if a is None else a.ctypes.data)
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    b = api.Batch(ctx, [dict(arm=wl.arm, p_spec=wl.p_spec, m2=wl.m2, sieve=1, seed=1, offset=0, count=n)])
+    assert L.simc_arm_run_fresh(ctx._h, wl.arm, C.byref(S), C.byref(ein), C.byref(eout), n, C.byref(R), st) == E_ARG
+    assert L.simc_arm_run_host_fresh(ctx._h, wl.arm, C.byref(S), C.byref(hin), C.byref(hout), n, C.byref(R)) == E_ARG
+    assert L.simc_batch_run_fresh(b._h, C.byref(ein), C.byref(eout), st) == E_ARG
+    torch.cuda.synchronize()
+    for k, v in dirty(n).items():
+        np.testing.assert_array_equal(new[k].cpu().numpy(), v, err_msg=k)
+        np.testing.assert_array_equal(got[k], v, err_msg=k)
