@@ -7,7 +7,8 @@ compile the HIP kernels (one unit per kernel family, in parallel), the output
 formats and the host map reader into one shared library;
 build the per-event Fortran-ABI drop-in libsimc_dropin.so on top of it; and,
 when a Fortran compiler is present, compile the Fortran module simc_gpu and
-the Fortran test programs of tests/fortran against both libraries.
+the Fortran test programs of tests/fortran against both libraries; compile
+the device functions that tests/device calls on arrays.
 """
 from __future__ import annotations
 
@@ -84,6 +85,7 @@ def build(verbose: bool = True) -> str:
     link(objs, verbose)
     build_dropin(verbose)
     build_fortran(verbose)
+    build_device_tests(verbose)
     return LIB
 
 
@@ -140,6 +142,20 @@ def build_fortran(verbose: bool = True) -> bool:
             print(" ".join(c))
         subprocess.run(c, check=True)
     return True
+
+
+def build_device_tests(verbose: bool = True) -> str:
+    """tests/device/_bin/libroot_helpers.so: device functions of the kernels
+    over arrays, for their tests."""
+    tdir = os.path.join(REPO, "tests", "device")
+    out = os.path.join(tdir, "_bin", "libroot_helpers.so")
+    os.makedirs(os.path.dirname(out), exist_ok=True)
+    cmd = [HIPCC, *HIP_FLAGS, "-shared", "-I", CSRC, os.path.join(tdir, "root_helpers.hip"), "-o", out + ".tmp"]
+    if verbose:
+        print(" ".join(cmd))
+    subprocess.run(cmd, check=True)
+    os.replace(out + ".tmp", out)
+    return out
 
 
 if __name__ == "__main__":
