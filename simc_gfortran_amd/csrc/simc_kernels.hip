@@ -1945,17 +1945,29 @@ __global__ __launch_bounds__(kFieldBlock) __attribute__((amdgpu_waves_per_eu(4))
 // dependent RK4 steps (3,300 of 1.4 us each for 1e5 HMS events, where the
 // mean is 580).  Two lanes per event: both run the reconstruction and the
 // long search (the same values), one each of the two searches to z = 0.
-// Events are dealt out over all wavefronts (event e to wavefront e mod the
-// number of wavefronts), so that few of them share a wavefront's loop.
-constexpr uint32_t kFinishEvents = 256 / 2;  // events a workgroup takes at once
+// The events are dealt out over one wavefront per CU, and over more only when
+// those hold 32 events each: wavefronts of a CU that are at different places
+// of the loop hold each other up.  Dealt over all wavefronts of the grid, 3,000
+// SOS events waited for instruction issue in 65 % of the wavefronts' cycles
+// (27 % for 10,000, five to a wavefront) and took longer than 10,000: 2.1 and
+// 1.2 ms, 0.8 and 0.8 dealt this way (HMS 4.9 and 4.4, 3.0 and 3.4; SHMS 3.6
+// and 3.1, 2.1 and 2.6; HRS 2.4 and 1.3, 0.9 and 0.9).
+constexpr uint32_t kFinishWave = 64 / 2;                    // events a wavefront takes at once
+constexpr uint32_t kFinishEvents = kFinishWave * 256 / 64;  // and a workgroup
+constexpr uint32_t kFinishPerCu = 2;                        // workgroups launched per CU
 
 // Rounds before field_to_finish for n events when it takes `cap` at once:
 // none where all fit, else as many as leave about one filling (of 1e5 HMS
 // events 97 % iterate after two rounds, 61, 29, 16 and 10 % after three to
-// six).  Measured in ms with 0, 3, 4, 5, 9 rounds (cap 65,536): 1e3 events
-// 3.6, 3.0, 3.1, 3.4, 4.9; 6e4: 5.5, 6.4, 6.8, 7.9, 9.3; 1e5: 7.9, 6.9, 8.1,
-// 9.9, 13.8; 2e5: 12.6, 9.7, 8.5, 10.0, 16.2; 7e5: -, 24.8, 19.7, 16.9, 18.8.
-// Ten rounds with the same search took 14.3 ms for the 1e5.
+// six).  Measured in ms with 0, 3, 4, 5, 9 rounds (cap 65,536):
+//   HMS   1e3 2.6, 2.9, 3.0, 3.4, 4.9    1e4 3.4, 3.7, 4.1, 4.4, 5.8    6.5e4 5.5, 6.2, 6.2, 6.5, 8.6
+//         1e5 7.5, 6.6, 6.9, 7.7, 13.2   2e5 12.1, 9.7, 8.7, 9.8, 15.1  7e5 31, 23.7, 19.8, 17.0, 18.4
+//   SHMS  1e3 2.0, 2.1, 2.2, 2.3, 2.9    1e4 2.6, 2.8, 3.1, 3.5, 5.0    6.5e4 3.7, 3.8, 4.0, 4.6, 7.5
+//         1e5 5.4, 4.3, 5.2, 5.8, 10.8   2e5 9.1, 7.1, 5.8, 8.0, 13.8   7e5 23, 15.7, 12.7, 12.9, 17.4
+// Ten rounds with the same search took 14.3 ms for the 1e5 HMS events.  SOS
+// and HRS events leave the loop within five iterations: at 1e4 and below none
+// is best as well (0.8 against 0.9 ms), from 2e4 to cap five rounds would take
+// 0.9-1.0 ms where none takes 1.1-1.3, above 2 cap the lines differ by 5 %.
 inline int field_rounds(uint64_t n, uint64_t cap) { return n <= cap ? 0 : n <= 2 * cap ? 3 : n <= 4 * cap ? 4 : 5; }
 
 template <int ARM>
@@ -1963,14 +1975,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 {
     __shared__ TrgNode s[kTrgStaged];
     const uint32_t count = *a.count_in;
-    const uint32_t n_waves = gridDim.x * (256u / 64u);
-    // wavefronts of a workgroup are numbered gridDim.x apart: the first events go to different CUs
+    const uint32_t full = (count + kFinishWave - 1u) / kFinishWave;
+    const uint32_t n_waves = min(gridDim.x * (256u / 64u), max(full, min(count, gridDim.x / kFinishPerCu)));
+    // wavefronts of a workgroup are numbered gridDim.x apart: the first ones go to different CUs
     const uint32_t wave = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-    if (blockIdx.x >= count) return;  // no event for any wavefront of this workgroup
+    if (blockIdx.x >= n_waves) return;  // no event for any wavefront of this workgroup
     stage_field_map(s, a.map);
+    if (wave >= n_waves) return;
     const TrgMap M{s, a.stht, a.ctht};
     const bool second = (threadIdx.x & 1u) != 0;
-    for (uint32_t e = wave + ((threadIdx.x & 63u) >> 1) * n_waves; e < count; e += 32u * n_waves) {
+    for (uint32_t e = wave + ((threadIdx.x & 63u) >> 1) * n_waves; e < count; e += kFinishWave * n_waves) {
         const uint32_t i = a.list_in[e];
         EvOut o, r;
         o.x_fp = a.x_fp[i];
@@ -3848,7 +3862,7 @@ int simc_track_to_tgt(simc_ctx* ctx, const simc_field* f, int arm, int spect, in
     a.list_out = list[0];
     a.count_out = count;
     hipLaunchKernelGGL(field_to_start, GS, BS, 0, st, a);
-    const uint32_t finish_grid = (uint32_t)f->n_cu * 2u;
+    const uint32_t finish_grid = (uint32_t)f->n_cu * kFinishPerCu;
     const int rounds = field_rounds((uint64_t)n, (uint64_t)finish_grid * kFinishEvents);
 #define FOR_ARM(KERNEL, GRID)                                                                              \
     do {                                                                                                   \

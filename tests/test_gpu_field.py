@@ -193,3 +193,25 @@ def test_to_tgt_same_for_any_number_of_events(ctx, n):
     for k in one:
         np.testing.assert_array_equal(all_[k], one[k][np.arange(n) % m], err_msg=k)
     F.close()
+
+
+@pytest.mark.parametrize("golden", ["to_hrsl_electron", "to_shms_electron"])
+@pytest.mark.parametrize("n", [31, 33, 1000, 16_385])
+def test_to_tgt_finish_deals_every_event_once(ctx, golden, n):
+    """The finishing kernel alone (no rounds before it), its wavefronts filled
+    with 32 events each: less than one, one and a bit, some of the workgroups,
+    one more wavefront than workgroups."""
+    from simc_gfortran_amd import api
+    g = np.load(os.path.join(HERE, "golden", "field", golden + ".npz"))
+    F = field_of(api, str(g["map"]), float(g["theta_e"]), float(g["theta_p"]))
+    m = len(g["mom"])
+    at = np.arange(n) % m
+    trk = {q: dev(g["trk_" + q][at]) for q in ("x_fp", "dx_fp", "y_fp", "dy_fp")}
+    rec = {q: dev(g["in_" + q][at]) for q in ("delta", "y", "dx", "dy")}
+    ok = F.track_to_tgt(ctx, int(g["arm"]), trk, rec, dev(g["frx"][at]), dev(g["fry"][at]), dev(g["mom"][at]),
+                        float(g["mass"]), float(g["ctheta"]), float(g["stheta"]), int(g["spect"]))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(ok.cpu().numpy(), g["out_ok"][at])
+    for q, sc in (("delta", 1.0), ("y", 1.0), ("dx", 1e-2), ("dy", 1e-2)):
+        assert close(rec[q].cpu().numpy(), g["out_" + q][at], sc).all(), q
+    F.close()
