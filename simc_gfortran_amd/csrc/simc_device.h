@@ -109,9 +109,11 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
 // Square root by one coupled (Goldschmidt) iteration from the hardware's
 // reciprocal square root (2^-24) and one residual correction (Markstein);
 // `y` receives 1 / sqrt(s) to 2^-47, enough for div_by's residual to round a
-// quotient.  Before their last rounding both results are within 2^-42 ulp;
-// for s in [2^-900, 2^1000] they equalled sqrt(s) and a / sqrt(s) on all of
-// 5e9 samples, without the scaling and special cases of the general forms.
+// quotient.  Before their last rounding both results are within 2^-42 ulp of
+// the exact ones, so one in about 2^42 may round the other way than sqrt(s) and
+// a / sqrt(s) (s in [2^-900, 2^1000]; no scaling and no special cases, as the
+// general forms have them).  The tests hold millions of them equal in each
+// range they are used in.
 __device__ __forceinline__ double sqrt_inv(double s, double& y)
 {
     const double y0 = __builtin_amdgcn_rsq(s);

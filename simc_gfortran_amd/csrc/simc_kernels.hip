@@ -891,11 +891,12 @@ __device__ __forceinline__ void count_slit(const KArgs& a, unsigned* hist, uint3
 // the hut stage, TO_Q lists the accepted events (index and setting) for
 // recon_list_kernel instead of reconstructing them here.
 // The common variants are held to three wavefronts per SIMD (168 VGPRs),
-// the hut stage to four (128 VGPRs: a few values may spill to scratch, and
-// the extra wavefront hides more of the hut's latency than the spills cost),
-// the RARE variants to two (256 VGPRs, a few spills; at one wavefront a pion
-// run with decay took 1.45 x as long, at three the spills cost more than the
-// wavefront gives).
+// the hut stage to four (128 VGPRs: the HMS spills 3 values, the others none;
+// with a key per lane HMS 7, SHMS 2, SOS 1; the extra wavefront hides more of
+// the hut's latency than that costs), the RARE variants to two (256 VGPRs and 2
+// to 34 values spilled in the first two stages, 185 and none in the hut; at one
+// wavefront a pion run with decay took 1.45 x as long, at three the spills cost
+// more than the wavefront gives).
 template <int ARM, class R, bool RARE, int STAGE, bool FROM_Q, bool TO_Q>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(RARE ? 2 : (STAGE == STAGE_HUT ? 4 : 3)))) void stage_kernel(
     KArgs a, Queue qin, Queue qout, int32_t pc_begin, int32_t pc_end)
@@ -1688,9 +1689,10 @@ struct GenRadArgs {
     int32_t* used;
 };
 
-// Held to three wavefronts per SIMD (168 VGPRs, about 260 values spilled):
-// at two (its unconstrained 276 registers) the kernel waited on its
-// elementary functions' latency and took 1.8 x as long.
+// Held to three wavefronts per SIMD (168 VGPRs, 472 values spilled to 528
+// bytes of scratch a lane): 1e3, 1e6 and 1e7 events take 0.175, 1.33 and 12.15
+// ms; at two (235 VGPRs, none spilled) 0.171, 1.40 and 13.13, at four (128,
+// 824 spilled) 0.186, 1.32 and 11.82.
 template <class R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void gen_hep_rad_kernel(GenRadArgs a)
 {

@@ -73,10 +73,11 @@ __device__ __noinline__ double rad_inter(double alpha, double ar1, double ar2, d
 }
 
 // gamma, out of line: the generator calls it 24 times, and with an inlined
-// copy at each the kernel was 739 KB of code, eleven times the instruction
-// cache (1e6 events: 1.46 -> 1.32 ms, fewer values in scratch, same bits).
-// Powers and logarithms out of line as well gave nothing more: the registers
-// saved around the calls cost what the code saves.
+// copy at each the kernel was 742 KB of code, eleven times the instruction
+// cache, now 538 (1e6 events: 1.44 -> 1.33 ms, 1e7: 13.2 -> 12.2, same bits).
+// The calls raise the values spilled from 282 to 472, the scratch falls from
+// 688 to 528 bytes a lane.  Powers and logarithms out of line as well gave
+// nothing more: the registers saved around the calls cost what the code saves.
 __device__ __noinline__ double rad_tgamma(double x) { return tgamma(x); }
 
 // inter_prime, brem.f:581-598
