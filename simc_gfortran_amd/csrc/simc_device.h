@@ -142,7 +142,7 @@ struct __attribute__((aligned(16))) BmLogEntry {
     float nlo, invc;
 };
 static __constant__ BmLogEntry kBmLogTab[SIMC_BM_LOG_N] = SIMC_BM_LOG_TABLE;
-static __constant__ double kBmSinCosTab[SIMC_BM_SINCOS_N][2] = SIMC_BM_SINCOS_TABLE;
+static __constant__ __attribute__((aligned(16))) double kBmSinCosTab[SIMC_BM_SINCOS_N][2] = SIMC_BM_SINCOS_TABLE;
 
 // A 16-byte table entry at byte offset `off` from a table in constant memory:
 // one load from a scalar base and a 32-bit lane offset.
